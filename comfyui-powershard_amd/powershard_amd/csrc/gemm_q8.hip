@@ -28,6 +28,7 @@
 // accumulators in registers and stages 32 x 64 blocks through LDS for whole-line stores while the
 // next tile's first stage loads.  MFMA-bound: 2 M N K ops per launch.
 #include "psq_common.hpp"
+#include "gemm_q8.hpp"
 
 namespace psq {
 namespace {
@@ -43,17 +44,6 @@ constexpr int LPS = 2 * LOADS;                       // ring loads per wave per 
 constexpr int GROUP_M = 8;                           // tile rows per raster group
 
 enum { OUT_BF16 = PSQ_BF16, OUT_F16 = PSQ_F16, OUT_F32 = PSQ_F32, OUT_I32 = 3 };
-
-struct Epi {
-    const float *a_scale;
-    const float *w_scale;
-    int w_per_row;
-    const void *bias;
-    int bias_dtype;
-    void *y;
-    int64_t ldy;
-    int vec;          // rows of y are 16-byte aligned: 4-element vector stores allowed
-};
 
 // Two outputs packed for a vector store (round to nearest even).
 template <int OUT>
@@ -214,14 +204,6 @@ __device__ __forceinline__ void tile_coords(int v, int nbm, int nbn, int &m0, in
     n0 = (r / h) * BN;
 }
 
-// Bias word (see above) to fp32.
-__device__ __forceinline__ float bias_word(uint32_t w, int dt)
-{
-    if (dt == PSQ_BF16) return __uint_as_float(w << 16);
-    if (dt == PSQ_F16) return f16_to_f32(w);
-    return __uint_as_float(w);
-}
-
 // Persistent kernel: one workgroup per CU walks its tiles; the LDS ring streams continuously
 // across tile boundaries, so the first stages of the next tile load while the current tile's
 // epilogue runs.  The MFMAs compute the transposed tile (W fragment as the first operand), which
@@ -231,7 +213,7 @@ __device__ __forceinline__ float bias_word(uint32_t w, int dt)
 template <bool FP8, int OUT, int ACT, int WF = 0>
 __global__ void __launch_bounds__(NTHREADS, 1)
 gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__restrict__ W, int64_t ldw,
-               int M, int N, int K, Epi ep)
+               int M, int N, int K, Q8Epi ep)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // ring A[NSTAGE] | W[NSTAGE], scales
     using Acc = typename std::conditional<FP8, v16f, v16i>::type;
@@ -949,7 +931,7 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
 
 template <bool FP8, int OUT, int ACT, int WF = 0>
 int launch_one(const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M, int64_t N, int64_t K,
-               const Epi &ep, hipStream_t st, const char *name)
+               const Q8Epi &ep, hipStream_t st, const char *name)
 {
     auto kern = gemm_q8_kernel<FP8, OUT, ACT, WF>;
     int dev = 0;
@@ -972,7 +954,7 @@ int launch_one(const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int
 
 template <bool FP8>
 int launch(int out, int act, const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M, int64_t N,
-           int64_t K, const Epi &ep, hipStream_t st, const char *name)
+           int64_t K, const Q8Epi &ep, hipStream_t st, const char *name)
 {
     if (act == ACT_SILU_GATE) {
         switch (out) {
@@ -1055,7 +1037,11 @@ int psq_gemm_i8_act(const int8_t *a, int64_t lda, const float *a_scale, const in
     if (!a_scale || !w_scale || !y) return set_error(PSQ_E_ARG, "gemm_i8: null scale or output");
     if (!valid_dtype(y_dtype) || (bias && !valid_dtype(bias_dtype))) return set_error(PSQ_E_ARG, "gemm_i8: bad dtype");
     if (int e = require_device()) return e;
-    Epi ep{a_scale, w_scale, 1, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_dtype == PSQ_F32 ? 4 : 2)};
+    Q8Epi ep{a_scale, w_scale, 1, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_dtype == PSQ_F32 ? 4 : 2)};
+    int status;
+    if (q8_small(Q8_I8, (const uint8_t *)a, lda, (const uint8_t *)w, ldw, M, N, K, ep, y_dtype, activation,
+                 (hipStream_t)stream, "gemm_i8", status))
+        return status;
     return launch<false>(y_dtype, activation, (const uint8_t *)a, lda, (const uint8_t *)w, ldw, M, N, K, ep,
                          (hipStream_t)stream, "gemm_i8");
 }
@@ -1077,7 +1063,7 @@ int psq_gemm_i8_i32(const int8_t *a, int64_t lda, const int8_t *w, int64_t ldw, 
     if (!c) return set_error(PSQ_E_ARG, "gemm_i8_i32: null output");
     if (ldc < N) return set_error(PSQ_E_SHAPE, "gemm_i8_i32: ldc < N");
     if (int e = require_device()) return e;
-    Epi ep{nullptr, nullptr, 0, nullptr, 0, c, ldc, vec_ok(c, ldc, 4)};
+    Q8Epi ep{nullptr, nullptr, 0, nullptr, 0, c, ldc, vec_ok(c, ldc, 4)};
     return launch<false>(OUT_I32, ACT_NONE, (const uint8_t *)a, lda, (const uint8_t *)w, ldw, M, N, K, ep,
                          (hipStream_t)stream, "gemm_i8_i32");
 }
@@ -1093,7 +1079,10 @@ int psq_gemm_fp8_act(const uint8_t *a, int64_t lda, const float *a_scale, const 
     if (!a_scale || !w_scale || !y) return set_error(PSQ_E_ARG, "gemm_fp8: null scale or output");
     if (!valid_dtype(y_dtype) || (bias && !valid_dtype(bias_dtype))) return set_error(PSQ_E_ARG, "gemm_fp8: bad dtype");
     if (int e = require_device()) return e;
-    Epi ep{a_scale, w_scale, w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_dtype == PSQ_F32 ? 4 : 2)};
+    Q8Epi ep{a_scale, w_scale, w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_dtype == PSQ_F32 ? 4 : 2)};
+    int status;
+    if (q8_small(Q8_E4M3, a, lda, w, ldw, M, N, K, ep, y_dtype, activation, (hipStream_t)stream, "gemm_fp8", status))
+        return status;
     return launch<true>(y_dtype, activation, a, lda, w, ldw, M, N, K, ep, (hipStream_t)stream, "gemm_fp8");
 }
 
@@ -1117,9 +1106,11 @@ int psq_gemm_fp8_e5m2w(const uint8_t *a, int64_t lda, const float *a_scale, cons
     if (!valid_dtype(y_dtype) || (bias && !valid_dtype(bias_dtype)))
         return set_error(PSQ_E_ARG, "gemm_fp8_e5m2w: bad dtype");
     if (int e = require_device()) return e;
-    Epi ep{a_scale, w_scale, w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_dtype == PSQ_F32 ? 4 : 2)};
+    Q8Epi ep{a_scale, w_scale, w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_dtype == PSQ_F32 ? 4 : 2)};
     hipStream_t st = (hipStream_t)stream;
     const char *name = "gemm_fp8_e5m2w";
+    int status;
+    if (q8_small(Q8_E5M2W, a, lda, w, ldw, M, N, K, ep, y_dtype, ACT_NONE, st, name, status)) return status;
     switch (y_dtype) {
     case OUT_BF16: return launch_one<true, OUT_BF16, ACT_NONE, 1>(a, lda, w, ldw, M, N, K, ep, st, name);
     case OUT_F16: return launch_one<true, OUT_F16, ACT_NONE, 1>(a, lda, w, ldw, M, N, K, ep, st, name);

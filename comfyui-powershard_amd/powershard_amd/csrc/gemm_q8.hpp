@@ -1,0 +1,36 @@
+// gemm_q8.hpp -- what the translation units of the W8A8 / FP8 GEMM share.
+#pragma once
+
+#include "psq_common.hpp"
+
+namespace psq {
+
+// Epilogue operands and output of a W8A8 / FP8 GEMM.
+struct Q8Epi {
+    const float *a_scale;
+    const float *w_scale;
+    int w_per_row;
+    const void *bias;
+    int bias_dtype;
+    void *y;
+    int64_t ldy;
+    int vec;          // rows of y are 16-byte aligned: 4-element vector stores allowed
+};
+
+// Operand kinds: int8 x int8, e4m3 x e4m3, e4m3 activations x e5m2 weights.
+enum { Q8_I8 = 0, Q8_E4M3 = 1, Q8_E5M2W = 2 };
+
+// Runs the problem on the small tiles (gemm_q8_small.hip) when they are the faster ones: true and its
+// status, or false and nothing launched.  Arguments as checked by the entry points.
+bool q8_small(int kind, const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M, int64_t N, int64_t K,
+              const Q8Epi &ep, int out, int act, hipStream_t st, const char *name, int &status);
+
+// A bias word (the bias element zero-extended, or the fp32 bits) to fp32.
+__device__ __forceinline__ float bias_word(uint32_t w, int dt)
+{
+    if (dt == PSQ_BF16) return __uint_as_float(w << 16);
+    if (dt == PSQ_F16) return f16_to_f32(w);
+    return __uint_as_float(w);
+}
+
+}  // namespace psq
