@@ -17,13 +17,30 @@ struct Q8Epi {
     int vec;          // rows of y are 16-byte aligned: 4-element vector stores allowed
 };
 
+// One checked call.
+struct Q8Args {
+    const uint8_t *a;
+    int64_t lda;
+    const uint8_t *w;
+    int64_t ldw, M, N, K;
+    Q8Epi ep;
+    hipStream_t st;
+    const char *name;
+};
+
 // Operand kinds: int8 x int8, e4m3 x e4m3, e4m3 activations x e5m2 weights.
 enum { Q8_I8 = 0, Q8_E4M3 = 1, Q8_E5M2W = 2 };
 
 // Runs the problem on the small tiles (gemm_q8_small.hip) when they are the faster ones: true and its
-// status, or false and nothing launched.  Arguments as checked by the entry points.
-bool q8_small(int kind, const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M, int64_t N, int64_t K,
-              const Q8Epi &ep, int out, int act, hipStream_t st, const char *name, int &status);
+// status, or false and nothing launched.
+bool q8_small(int kind, int out, int act, const Q8Args &x, int &status);
+
+// The large tiles: 256 x 256 (every output and activation of its kind; out 3 = int32, int8 only), and
+// 256 x width, width 224, 192 or 160 (bf16 / f16 outputs, no gate).
+int q8_square_i8(int out, int act, const Q8Args &x);
+int q8_square_fp8(int kind, int out, int act, const Q8Args &x);
+int q8_width_i8(int width, int out, int act, const Q8Args &x);
+int q8_width_fp8(int kind, int width, int out, int act, const Q8Args &x);
 
 // A bias word (the bias element zero-extended, or the fp32 bits) to fp32.
 __device__ __forceinline__ float bias_word(uint32_t w, int dt)

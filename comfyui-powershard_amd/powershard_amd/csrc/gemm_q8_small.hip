@@ -366,23 +366,22 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
 }
 
 template <int KIND, int NW, int TM, int TN, int NRG, int NCG, int RA, int BUDGET, bool PIPE, bool GATE>
-int launch_cfg(const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M, int64_t N, int64_t K,
-               const Q8Epi &ep, int out, int act, hipStream_t st, const char *name)
+int launch_cfg(int out, int act, const Q8Args &x)
 {
     using C = Cfg<NW, TM, TN, NRG, NCG, RA, BUDGET>;
     auto kern = q8_small_kernel<KIND, NW, TM, TN, NRG, NCG, RA, BUDGET, PIPE, GATE>;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return set_error(PSQ_E_DEVICE, "%s: no device", name);
+    if (hipGetDevice(&dev) != hipSuccess) return set_error(PSQ_E_DEVICE, "%s: no device", x.name);
     static bool attr_set[64] = {};   // per device; the attribute is idempotent
     if (dev >= 64 || !attr_set[dev]) {
         if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::SMEM) != hipSuccess)
-            return set_error(PSQ_E_DEVICE, "%s: cannot reserve %d bytes of LDS", name, C::SMEM);
+            return set_error(PSQ_E_DEVICE, "%s: cannot reserve %d bytes of LDS", x.name, C::SMEM);
         if (dev < 64) attr_set[dev] = true;
     }
-    const int64_t NO = GATE ? N / 2 : N, on = GATE ? C::BN / 2 : C::BN;
-    const int64_t tiles = ((M + C::BM - 1) / C::BM) * ((NO + on - 1) / on);
-    kern<<<dim3((unsigned)tiles), dim3(64 * NW), C::SMEM, st>>>(a, lda, w, ldw, (int)M, (int)N, (int)K, ep, out, act);
-    return check_launch(name);
+    const int64_t NO = GATE ? x.N / 2 : x.N, on = GATE ? C::BN / 2 : C::BN;
+    const int64_t tiles = ((x.M + C::BM - 1) / C::BM) * ((NO + on - 1) / on);
+    kern<<<dim3((unsigned)tiles), dim3(64 * NW), C::SMEM, x.st>>>(x.a, x.lda, x.w, x.ldw, (int)x.M, (int)x.N, (int)x.K, x.ep, out, act);
+    return check_launch(x.name);
 }
 
 // The tile shapes: rows x W rows, the waves' split of them and of K, and whether a tile's fragments
@@ -423,11 +422,10 @@ int pick_shape(bool gate, int64_t M, int64_t N, int cus)
 }
 
 template <int KIND>
-int launch_shape(int shape, bool gate, const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M,
-                 int64_t N, int64_t K, const Q8Epi &ep, int out, int act, hipStream_t st, const char *name)
+int launch_shape(int shape, bool gate, int out, int act, const Q8Args &x)
 {
     constexpr int KB = 1024;
-#define PSQ_GO(...) return launch_cfg<KIND, __VA_ARGS__>(a, lda, w, ldw, M, N, K, ep, out, act, st, name)
+#define PSQ_GO(...) return launch_cfg<KIND, __VA_ARGS__>(out, act, x)
     if (gate) {
         if constexpr (KIND != 2) {
             switch (shape) {
@@ -439,7 +437,7 @@ int launch_shape(int shape, bool gate, const uint8_t *a, int64_t lda, const uint
             default: PSQ_GO(8, 4, 4, 4, 2, 0, 156 * KB, true, true);
             }
         }
-        return set_error(PSQ_E_ARG, "%s: no gate for these weights", name);
+        return set_error(PSQ_E_ARG, "%s: no gate for these weights", x.name);
     }
     switch (shape) {
     case T16x32: PSQ_GO(8, 1, 1, 1, 2, 0, 76 * KB, false, false);
@@ -456,18 +454,17 @@ int launch_shape(int shape, bool gate, const uint8_t *a, int64_t lda, const uint
 
 }  // namespace
 
-bool q8_small(int kind, const uint8_t *a, int64_t lda, const uint8_t *w, int64_t ldw, int64_t M, int64_t N, int64_t K,
-              const Q8Epi &ep, int out, int act, hipStream_t st, const char *name, int &status)
+bool q8_small(int kind, int out, int act, const Q8Args &x, int &status)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return false;   // the caller's launch reports it
     const bool gate = act == ACT_SILU_GATE;
-    const int shape = pick_shape(gate, M, N, cu_count(dev));
+    const int shape = pick_shape(gate, x.M, x.N, cu_count(dev));
     if (shape < 0) return false;
     switch (kind) {
-    case Q8_I8: status = launch_shape<0>(shape, gate, a, lda, w, ldw, M, N, K, ep, out, act, st, name); break;
-    case Q8_E4M3: status = launch_shape<1>(shape, gate, a, lda, w, ldw, M, N, K, ep, out, act, st, name); break;
-    default: status = launch_shape<2>(shape, gate, a, lda, w, ldw, M, N, K, ep, out, act, st, name); break;
+    case Q8_I8: status = launch_shape<0>(shape, gate, out, act, x); break;
+    case Q8_E4M3: status = launch_shape<1>(shape, gate, out, act, x); break;
+    default: status = launch_shape<2>(shape, gate, out, act, x); break;
     }
     return true;
 }
