@@ -246,8 +246,8 @@ gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int
 }
 
 // ------------------------------------------------------------------ tiled kernel (M > 64)
-// A BM x 256 output tile (BM = 256, or 128 when that fills more of the GPU) per workgroup of 8
-// waves, two per SIMD.  Wave w owns all BM rows (tokens) and the 32 weight rows (output columns)
+// A BM x 256 output tile (BM = 128 to 256 in steps of 32, plan_tiled) per workgroup of 8 waves, two
+// per SIMD.  Wave w owns all BM rows (tokens) and the 32 weight rows (output columns)
 // 32w .. 32w + 31: BM/32 MFMA tiles of 32 x 32 on v_mfma_f32_32x32x16_bf16 / f16 with the
 // accumulators in AGPRs.  So every weight element is dequantized once per workgroup, by the one
 // wave that multiplies it, for BM rows.  Two waves per SIMD because the dequantization is VALU
@@ -271,7 +271,7 @@ constexpr int NWAVE = BN / WCOLS;                  // waves per workgroup (8: tw
 constexpr int THREADS = NWAVE * 64;
 constexpr int XROW = BK * 2;                       // activation bytes per row per stage
 template <int BM> constexpr int xbytes() { return BM * XROW; }                        // 32 / 16 KB
-template <int BM> constexpr int xdma() { return xbytes<BM>() / 1024 / NWAVE; }        // activation loads per wave (4 / 2)
+template <int BM> constexpr int xdma() { return (xbytes<BM>() / 1024 + NWAVE - 1) / NWAVE; }   // activation loads per wave
 template <int WK> constexpr int wrow() { return WK == W_UINT4 ? BK / 2 : BK; }         // 32 / 64 B
 template <int WK> constexpr int wdma() { return BN * wrow<WK>() / 1024 / NWAVE; }      // 1 / 2
 template <int WK> constexpr int szdma() { return WK == W_UINT4 ? 1 : 0; }
@@ -374,7 +374,8 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
         uint32_t xo[XDMA], wo[WDMA];
 #pragma unroll
         for (int j = 0; j < XDMA; j++) {
-            const int b = j * NWAVE + wave, r = 8 * b + (lane >> 3);
+            const int b = min(j * NWAVE + wave, BM / 8 - 1);   // (a block loaded twice holds the same bytes)
+            const int r = 8 * b + (lane >> 3);
             const int c = (lane & 7) ^ xsw(r);
             xo[j] = (uint32_t)(min(r, M - 1 - m0) * ldx * 2 + c * 16);
         }
@@ -410,8 +411,8 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
             constexpr int q = decltype(qc)::value;
             uint8_t *sl = smem + slot * SLOT;
             if constexpr (q < XDMA) {
-                constexpr int b8 = q * NWAVE;
-                buffer_load_lds16(rsx, (lds_ptr)(sl + 1024 * (b8 + wave)), xo[q], kt * BK * 2);
+                const int b = BM % (8 * NWAVE) ? min(q * NWAVE + wave, BM / 8 - 1) : q * NWAVE + wave;
+                buffer_load_lds16(rsx, (lds_ptr)(sl + 1024 * b), xo[q], kt * BK * 2);
             } else if constexpr (q < XDMA + WDMA) {
                 constexpr int j = q - XDMA;
                 buffer_load_lds16(rsw, (lds_ptr)(sl + XBYTES + 1024 * (j * NWAVE + wave)), wo[j], kt * RB);
@@ -548,11 +549,12 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                     constexpr int q = Q;
                     mfma(q / TN, q % TN, wc[q % TN], xc[q / TN]);
                     if constexpr (q % TN == 0) xn[q / TN] = read_x(xslot, tn, q / TN);
-                    // weight pair pi (column tile pi / 4, pair pi % 4), spread evenly over the k-step
-                    constexpr int NP = 4 * TN, PSTRIDE = NQ / NP;
-                    static_assert(NQ % NP == 0, "pairs per k-step must divide the MFMAs");
-                    constexpr int pi = q % PSTRIDE == 0 ? q / PSTRIDE : -1;
-                    if constexpr (pi >= 0) hw[pi >> 2][pi & 3] = dq_pair(wraw, pi >> 2, tn, pi & 3);
+                    // weight pairs (pair pi: column tile pi / 4, pair pi % 4), spread evenly over the k-step
+                    constexpr int NP = 4 * TN, p0 = (q * NP + NQ - 1) / NQ, p1 = ((q + 1) * NP + NQ - 1) / NQ;
+                    static_for<p1 - p0>([&](auto pc) {
+                        constexpr int pi = p0 + decltype(pc)::value;
+                        hw[pi >> 2][pi & 3] = dq_pair(wraw, pi >> 2, tn, pi & 3);
+                    });
                     // the refill loads: LPK of them spread over the k-step, the last of each group
                     constexpr int per = NQ / LPK, u = q / per;
                     if constexpr (fill_base >= 0 && q % per == per - 1 && u < LPK && fill_base + u < LPS)
@@ -1791,22 +1793,32 @@ int launch_tiled_bm(const uint16_t *x, int64_t ldx, int64_t M, int64_t N, int64_
 }
 
 // Launch plan of the tiled kernel, in units of one 128-row tile's K stage on a lightly loaded GPU.
-//  * Data-parallel (one tile per workgroup): ceil(tiles / CUs) rounds of nk stages; a 256-row
-//    tile's stage costs about kBm256Cost of a 128-row one (the dequantization serves twice the
-//    rows: at N=25600 x K=5120, 126 us for a 256-row tile against 78 for a 128-row one).
+//  * Data-parallel (one tile per workgroup): ceil(tiles / CUs) rounds of nk stages.  Tiles are 128,
+//    160, 192, 224 or 256 rows; a stage of theirs costs kRows[] of a 128-row one's (the
+//    dequantization serves all the rows: us a stage on 100 CUs, uint4, 0.86, 0.97, 1.02, 1.15, 1.25).
+//    The width in rows is the cheapest over the rounds it takes, so that a ragged M does not compute
+//    a mostly empty row tile: 300 x 25600 x 5120 125.1 us with two 256-row tiles, 93.0 with two of 160;
+//    384 x 25600 x 5120 127.5 -> 104.8 (192); 2048 x 25600 x 5120 529 -> 503 (224); f16 on int8 weights
+//    2048 x 5120 x 5120 109.2 -> 100.3 (192).
 //  * Stream-K, 128-row tiles only (the 256-row kernel has no registers to spare for it), over G
 //    workgroups: ceil(tiles nk / G) stages each.  With G a multiple s of the tiles, each workgroup
 //    takes one K range of one tile (one partial, written or added up); otherwise up to two
 //    segments (a second ring prologue, two partials).  Each partial costs about kSkPartCost.
 //  * The kernel is power-limited: with more than about 78% of the CUs busy the clock drops, a
 //    stage taking about 1 + 0.6 (busy fraction - 0.78) times as long (M=128 x N=25600: 1.13 us a
-//    stage on 200 CUs, 1.2-1.37 on 256).
+//    stage on 200 CUs, 1.2-1.37 on 256).  f16 on int8 weights has so little dequantization that
+//    a stage on 160 CUs takes 0.75 us against 1.13 of stream-K on 256 (kSkStageF16I8): 1024 x 5120 x
+//    5120 64.6 us with stream-K, 59.7 with 160 whole tiles.
 // Stream-K is taken when it beats data-parallel by more than kSkMargin, and needs a workspace:
 // the tiles' arrival counters (kSkCntBytes, room for kSkMaxTiles) and two fp32 partial tiles per
-// workgroup.  Without stream-K, 128-row tiles while they fit one round of workgroups.
+// workgroup.
 constexpr int kSkMinUnits = 8;                              // K stages per workgroup at least
 constexpr double kSkPartCost = 3.0, kSkRestartCost = 2.0, kSkMargin = 0.9;
-constexpr double kBm256Cost = 1.4;
+constexpr struct {
+    int bm;
+    double cost;
+} kRows[] = {{128, 1.0}, {160, 1.10}, {192, 1.17}, {224, 1.32}, {256, 1.44}};
+constexpr double kSkStageF16I8 = 1.4;
 constexpr int64_t kSkMaxTiles = 16384;
 constexpr int64_t kSkCntBytes = kSkMaxTiles * 4;
 constexpr int64_t kSkSlotBytes = 128LL * wt::BN * 4;        // one 128-row fp32 partial tile
@@ -1826,22 +1838,27 @@ struct TiledPlan {
     int64_t ws_bytes = 0;
 };
 
-TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, int cus, bool allow_sk)
+TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, int cus, bool allow_sk, double sk_stage = 1.0)
 {
     TiledPlan p;
     const int64_t nbn = (N + wt::BN - 1) / wt::BN, nk = K / wt::BK;
-    p.bm = ((M + 127) / 128) * nbn <= cus ? 128 : 256;
-    p.tiles = ((M + p.bm - 1) / p.bm) * nbn;
+    double t_dp = 0.0;
+    for (const auto &r : kRows) {
+        const int64_t tiles = ((M + r.bm - 1) / r.bm) * nbn;
+        const double t = (double)((tiles + cus - 1) / cus * nk) * r.cost * clock_factor(std::min<int64_t>(tiles, cus), cus);
+        if (p.tiles && t >= t_dp) continue;
+        t_dp = t;
+        p.bm = r.bm;
+        p.tiles = tiles;
+    }
     if (!allow_sk) return p;
-    const double t_dp = (double)((p.tiles + cus - 1) / cus * nk) * (p.bm == 256 ? kBm256Cost : 1.0) *
-                        clock_factor(std::min<int64_t>(p.tiles, cus), cus);
     const int64_t t128 = ((M + 127) / 128) * nbn, units = t128 * nk;
     if (t128 > kSkMaxTiles) return p;
     double best = kSkMargin * t_dp;
     int64_t best_g = 0;
     auto consider = [&](int64_t g, bool aligned) {
         if (g < 1 || g > cus || g > kSkMaxGroups || units / g < kSkMinUnits) return;
-        const double t = (double)((units + g - 1) / g) * clock_factor(g, cus) +
+        const double t = (double)((units + g - 1) / g) * clock_factor(g, cus) * sk_stage +
                          (aligned ? kSkPartCost : 2 * kSkPartCost + kSkRestartCost);
         if (t < best) {
             best = t;
@@ -1927,7 +1944,8 @@ int launch(const void *x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_
     }
     if (ldx > (1LL << 22)) return set_error(PSQ_E_SHAPE, "%s: ldx above 2^22", name);   // 32-bit row offsets
     if (K > (1LL << 22)) return set_error(PSQ_E_SHAPE, "%s: K above 2^22", name);       // (of the weights too)
-    const TiledPlan plan = plan_tiled(M, N, K, cu_count(dev), workspace != nullptr);
+    const TiledPlan plan = plan_tiled(M, N, K, cu_count(dev), workspace != nullptr,
+                                      WK == W_INT8 && x_dtype == PSQ_F16 ? kSkStageF16I8 : 1.0);
     wa.sk = 0;
     if (plan.sk) {
         if (ws_bytes < plan.ws_bytes)
@@ -1941,8 +1959,13 @@ int launch(const void *x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_
     auto go = [&](auto xc) {
         constexpr int XDT = decltype(xc)::value;
         if (plan.sk) return launch_tiled_bm<XDT, WK, 128, true>(xp, ldx, M, N, K, wa, st, name);
-        return plan.bm == 128 ? launch_tiled_bm<XDT, WK, 128, false>(xp, ldx, M, N, K, wa, st, name)
-                              : launch_tiled_bm<XDT, WK, 256, false>(xp, ldx, M, N, K, wa, st, name);
+        switch (plan.bm) {
+        case 128: return launch_tiled_bm<XDT, WK, 128, false>(xp, ldx, M, N, K, wa, st, name);
+        case 160: return launch_tiled_bm<XDT, WK, 160, false>(xp, ldx, M, N, K, wa, st, name);
+        case 192: return launch_tiled_bm<XDT, WK, 192, false>(xp, ldx, M, N, K, wa, st, name);
+        case 224: return launch_tiled_bm<XDT, WK, 224, false>(xp, ldx, M, N, K, wa, st, name);
+        default: return launch_tiled_bm<XDT, WK, 256, false>(xp, ldx, M, N, K, wa, st, name);
+        }
     };
     return x_dtype == PSQ_BF16 ? go(std::integral_constant<int, PSQ_BF16>{}) : go(std::integral_constant<int, PSQ_F16>{});
 }
