@@ -18,6 +18,7 @@ ABI_VERSION = 1
 
 BF16, F16, F32 = 0, 1, 2
 W_UINT4, W_INT8 = 0, 1   # enum psq_weight_kind
+Q8_I8, Q8_E4M3, Q8_E5M2 = 0, 1, 2   # enum psq_q8_weights
 
 # Every exported entry point: name -> (restype, argtypes).  Mirrors include/psquant.h.
 _P, _I64, _I = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
@@ -35,6 +36,8 @@ SIGNATURES = {
     "psq_gemm_fp8": (_I, [_P, _I64, _P, _P, _I64, _P, _I, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_fp8_e5m2w": (_I, [_P, _I64, _P, _P, _I64, _P, _I, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_fp8_act": (_I, [_P, _I64, _P, _P, _I64, _P, _I, _P, _I, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
+    "psq_linear_q8_scratch_bytes": (_I64, [_I64, _I64]),
+    "psq_linear_q8": (_I, [_I, _P, _I, _I64, _I, _P, _I64, _P, _I, _P, _I, _I, _P, _I64, _I64, _I64, _I64, _P, _P]),
     "psq_gemm_w4a16": (_I, [_P, _I, _I64, _P, _P, _P, _I, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_w8a16": (_I, [_P, _I, _I64, _P, _P, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_wonly_workspace_bytes": (_I64, [_I, _I64, _I64, _I64, _I64, _I]),

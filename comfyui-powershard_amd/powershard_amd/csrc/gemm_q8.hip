@@ -170,4 +170,35 @@ int psq_gemm_fp8_e5m2w(const uint8_t *a, int64_t lda, const float *a_scale, cons
     return run(Q8_E5M2W, y_dtype, ACT_NONE, {a, lda, w, ldw, M, N, K, ep, (hipStream_t)stream, "gemm_fp8_e5m2w"});
 }
 
+// The codes, rounded up to a 16-byte line, then the row scales.
+int64_t psq_linear_q8_scratch_bytes(int64_t M, int64_t K) { return M <= 0 || K <= 0 ? 0 : ((M * K + 15) & ~15LL) + 4 * M; }
+
+int psq_linear_q8(int weights, const void *x, int x_dtype, int64_t ldx, int rot_group, const void *w, int64_t ldw,
+                  const float *w_scale, int w_scale_per_row, const void *bias, int bias_dtype, int activation, void *y,
+                  int64_t ldy, int64_t M, int64_t N, int64_t K, void *scratch, void *stream)
+{
+    using namespace psq;
+    if (weights < PSQ_Q8_I8 || weights > PSQ_Q8_E5M2) return set_error(PSQ_E_ARG, "linear_q8: bad weights %d", weights);
+    if (weights == PSQ_Q8_E5M2 && activation != PSQ_ACT_NONE)
+        return set_error(PSQ_E_ARG, "linear_q8: e5m2 weights take no activation");
+    if (weights != PSQ_Q8_I8 && rot_group) return set_error(PSQ_E_ARG, "linear_q8: the rotation is int8's");
+    if (M > 0 && N > 0 && K > 0 && (!scratch || ((uintptr_t)scratch & 15)))
+        return set_error(PSQ_E_ARG, "linear_q8: scratch must be 16-byte aligned");
+    // refuse before the quantizer runs what the GEMM would refuse
+    if (int e = check_shapes("linear_q8", scratch, K, w, ldw, M, N, K)) return e;
+    uint8_t *q = (uint8_t *)scratch;
+    float *sx = (float *)(q + ((M * K + 15) & ~15LL));
+    if (weights == PSQ_Q8_I8) {
+        if (int e = psq_quantize_rows_i8(x, x_dtype, M, K, ldx, rot_group, nullptr, (int8_t *)q, K, sx, stream)) return e;
+        return psq_gemm_i8_act((const int8_t *)q, K, sx, (const int8_t *)w, ldw, w_scale, bias, bias_dtype, activation, y,
+                               x_dtype, ldy, M, N, K, stream);
+    }
+    if (int e = psq_quantize_rows_fp8(x, x_dtype, M, K, ldx, 0, nullptr, q, K, sx, stream)) return e;
+    if (weights == PSQ_Q8_E5M2)
+        return psq_gemm_fp8_e5m2w(q, K, sx, (const uint8_t *)w, ldw, w_scale, w_scale_per_row, bias, bias_dtype, y,
+                                  x_dtype, ldy, M, N, K, stream);
+    return psq_gemm_fp8_act(q, K, sx, (const uint8_t *)w, ldw, w_scale, w_scale_per_row, bias, bias_dtype, activation, y,
+                            x_dtype, ldy, M, N, K, stream);
+}
+
 }  // extern "C"

@@ -46,6 +46,8 @@ EXTRAS = ("pre_quant_scale", "input_scale")
 # Formats with a native kernel here and the library op that runs them.
 NATIVE = {"int8_tensorwise": "gemm_i8", "float8_e4m3fn": "gemm_fp8", "float8_e5m2": "gemm_fp8",
           "int4_asym_group": "gemm_w4a16"}
+# stored code type -> the library's weight kind (enum psq_q8_weights)
+_Q8_WEIGHTS = {torch.int8: 0, torch.float8_e4m3fn: 1, torch.float8_e5m2: 2}
 # The exceptions of a native attempt that switch a module to dequantize (quant_linear.py:207-215).
 NATIVE_FAILURES = (NotImplementedError, RuntimeError, TypeError, ValueError)
 
@@ -327,7 +329,65 @@ class QuantLinear(nn.Module):
             tracker.observe(self._ps_finite_slot, out)
         return out
 
+    def _direct(self, x, activation):
+        """The native forward in one library call, or None where anything has to be converted,
+        copied, shared, tracked, timed or refused: the general path below takes those (and reports
+        what the library refuses).  Same kernels, same values."""
+        own = self.__dict__
+        dtype = self._ps_compute_dtype
+        if (not self._ps_native or self._ps_full_precision or type(x) is not torch.Tensor or not x.is_cuda
+                or x.dtype is not dtype or (dtype is not torch.bfloat16 and dtype is not torch.float16)
+                or self._modules or own.get("_ps_safe") or own.get("_ps_tracker") is not None
+                or getattr(_shared, "cache", None) is not None):
+            return None
+        from . import ops
+        plan, store, bias = self._ps_qplan, self.qbytes, self.bias
+        layout, uint4 = plan.layout, plan.layout is qtm.UInt4GroupLayout
+        if len(plan.specs) != (3 if uint4 else 2):   # extras: the general path
+            return None
+        _, code, (N, K), q_at, _ = plan.specs[0]
+        name, sdtype, _, s_at, s_bytes = plan.specs[1]
+        if uint4:
+            K *= 2
+        numel, device = x.numel(), x.device
+        if (not numel or x.shape[-1] != K or not x.is_contiguous() or name != "scale" or store.device != device
+                or store.dtype is not torch.uint8 or store.dim() != 1 or store.numel() < plan.total
+                or not store.is_contiguous() or not ops.direct_available()):
+            return None
+        base, M = store.data_ptr(), numel // K
+        if (base | x.data_ptr()) % 16 or (bias is not None and (
+                bias.dtype is not dtype or bias.device != device or bias.numel() != N or not bias.is_contiguous())):
+            return None
+        if uint4:
+            name, zdtype, _, z_at, z_bytes = plan.specs[2]
+            group = plan.fields["group_size"]
+            if (activation is not None or name != "zero" or sdtype is not torch.float16 or zdtype is not torch.float16
+                    or K % group or s_bytes != 2 * N * (K // group) or z_bytes != s_bytes):
+                return None
+            return ops.linear_w4a16_direct(x, M, K, base + q_at, base + s_at, base + z_at, group, N, bias)
+        weights, count, rot = _Q8_WEIGHTS.get(code), s_bytes // 4, 0
+        if (weights is None or sdtype is not torch.float32 or (activation is not None and weights == 2)
+                or (activation == "silu_gate" and N % 128)):
+            return None
+        if layout is qtm.Int8RowwiseLayout:
+            if count != N or weights:
+                return None
+            if plan.fields["convrot"]:
+                rot = plan.fields["convrot_groupsize"]
+        elif layout is not qtm.Float8ScaledLayout or not weights or (count != N and count != 1):
+            return None
+        return ops.linear_q8_direct(x, M, K, weights, base + q_at, base + s_at, int(count > 1), rot, N, bias,
+                                    ops.ACTIVATIONS[activation])
+
     def _forward(self, x, activation):
+        try:
+            out = self._direct(x, activation)
+        except torch.cuda.OutOfMemoryError:
+            raise
+        except NATIVE_FAILURES:   # e.g. a tensor without storage (vmap): the general path's policy applies
+            out = None
+        if out is not None:
+            return out
         dtype = self._dtype_for(x)
         qt, extras = unpack(self.qbytes, self._ps_qplan, dtype, with_extras=True)
         rows = x.reshape(-1, x.shape[-1]).to(dtype)
