@@ -37,7 +37,7 @@ SIGNATURES = {
     "psq_gemm_fp8_e5m2w": (_I, [_P, _I64, _P, _P, _I64, _P, _I, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_fp8_act": (_I, [_P, _I64, _P, _P, _I64, _P, _I, _P, _I, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_linear_q8_scratch_bytes": (_I64, [_I64, _I64]),
-    "psq_linear_q8": (_I, [_I, _P, _I, _I64, _I, _P, _I64, _P, _I, _P, _I, _I, _P, _I64, _I64, _I64, _I64, _P, _P]),
+    "psq_linear_q8": (_I, [_I, _P, _I, _I64, _I, _P, _I64, _P, _I, _P, _I, _I, _P, _I, _I64, _I64, _I64, _I64, _P, _P]),
     "psq_gemm_w4a16": (_I, [_P, _I, _I64, _P, _P, _P, _I, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_w8a16": (_I, [_P, _I, _I64, _P, _P, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P]),
     "psq_gemm_wonly_workspace_bytes": (_I64, [_I, _I64, _I64, _I64, _I64, _I]),

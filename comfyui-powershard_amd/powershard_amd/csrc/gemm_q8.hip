@@ -6,10 +6,10 @@ namespace psq {
 namespace {
 
 // Vector stores need 16-byte-aligned rows; the staged stores also address a 32-row block with a
-// 32-bit lane offset, which holds for ldy < 2^26.  Other outputs take the element-store path.
+// 32-bit lane offset, which holds for rows below 2^27 bytes.  Other outputs take the element-store path.
 int vec_ok(const void *y, int64_t ldy, int elem)
 {
-    return (((uintptr_t)y & 15) == 0 && (ldy * elem) % 16 == 0 && ldy < (1LL << 26)) ? 1 : 0;
+    return (((uintptr_t)y & 15) == 0 && (ldy * elem) % 16 == 0 && ldy * elem < (1LL << 27)) ? 1 : 0;
 }
 
 int check_shapes(const char *name, const void *a, int64_t lda, const void *w, int64_t ldw, int64_t M, int64_t N,
@@ -129,7 +129,7 @@ int psq_gemm_i8_i32(const int8_t *a, int64_t lda, const int8_t *w, int64_t ldw, 
     if (ldc < N) return set_error(PSQ_E_SHAPE, "gemm_i8_i32: ldc < N");
     if (int e = require_device()) return e;
     Q8Epi ep{nullptr, nullptr, 0, nullptr, 0, c, ldc, vec_ok(c, ldc, 4)};
-    return q8_square_i8(3, ACT_NONE, {(const uint8_t *)a, lda, (const uint8_t *)w, ldw, M, N, K, ep,
+    return q8_square_i8(Q8_OUT_I32, ACT_NONE, {(const uint8_t *)a, lda, (const uint8_t *)w, ldw, M, N, K, ep,
                                       (hipStream_t)stream, "gemm_i8_i32"});
 }
 
@@ -175,30 +175,34 @@ int64_t psq_linear_q8_scratch_bytes(int64_t M, int64_t K) { return M <= 0 || K <
 
 int psq_linear_q8(int weights, const void *x, int x_dtype, int64_t ldx, int rot_group, const void *w, int64_t ldw,
                   const float *w_scale, int w_scale_per_row, const void *bias, int bias_dtype, int activation, void *y,
-                  int64_t ldy, int64_t M, int64_t N, int64_t K, void *scratch, void *stream)
+                  int y_f32, int64_t ldy, int64_t M, int64_t N, int64_t K, void *scratch, void *stream)
 {
     using namespace psq;
-    if (weights < PSQ_Q8_I8 || weights > PSQ_Q8_E5M2) return set_error(PSQ_E_ARG, "linear_q8: bad weights %d", weights);
-    if (weights == PSQ_Q8_E5M2 && activation != PSQ_ACT_NONE)
-        return set_error(PSQ_E_ARG, "linear_q8: e5m2 weights take no activation");
-    if (weights != PSQ_Q8_I8 && rot_group) return set_error(PSQ_E_ARG, "linear_q8: the rotation is int8's");
+    const char *name = "linear_q8";
+    if (weights < PSQ_Q8_I8 || weights > PSQ_Q8_E5M2) return set_error(PSQ_E_ARG, "%s: bad weights %d", name, weights);
+    if (weights == PSQ_Q8_E5M2 && (activation != PSQ_ACT_NONE || y_f32))
+        return set_error(PSQ_E_ARG, "%s: e5m2 weights take no activation and no fp32 output", name);
+    if (y_f32 && activation != PSQ_ACT_NONE) return set_error(PSQ_E_ARG, "%s: an activation has no fp32 output", name);
+    if (weights != PSQ_Q8_I8 && rot_group) return set_error(PSQ_E_ARG, "%s: the rotation is int8's", name);
+    if (x_dtype != PSQ_BF16 && x_dtype != PSQ_F16) return set_error(PSQ_E_ARG, "%s: activations must be bf16/f16", name);
+    if (bias && !valid_dtype(bias_dtype)) return set_error(PSQ_E_ARG, "%s: bad dtype", name);
     if (M > 0 && N > 0 && K > 0 && (!scratch || ((uintptr_t)scratch & 15)))
-        return set_error(PSQ_E_ARG, "linear_q8: scratch must be 16-byte aligned");
+        return set_error(PSQ_E_ARG, "%s: scratch must be 16-byte aligned", name);
     // refuse before the quantizer runs what the GEMM would refuse
-    if (int e = check_shapes("linear_q8", scratch, K, w, ldw, M, N, K)) return e;
+    if (int e = check_shapes(name, scratch, K, w, ldw, M, N, K)) return e;
+    if (int e = check_act(name, activation, N, ldw, K, ldy)) return e;
+    if (M == 0 || N == 0) return PSQ_OK;
+    if (!w_scale || !y) return set_error(PSQ_E_ARG, "%s: null scale or output", name);
     uint8_t *q = (uint8_t *)scratch;
     float *sx = (float *)(q + ((M * K + 15) & ~15LL));
-    if (weights == PSQ_Q8_I8) {
-        if (int e = psq_quantize_rows_i8(x, x_dtype, M, K, ldx, rot_group, nullptr, (int8_t *)q, K, sx, stream)) return e;
-        return psq_gemm_i8_act((const int8_t *)q, K, sx, (const int8_t *)w, ldw, w_scale, bias, bias_dtype, activation, y,
-                               x_dtype, ldy, M, N, K, stream);
-    }
-    if (int e = psq_quantize_rows_fp8(x, x_dtype, M, K, ldx, 0, nullptr, q, K, sx, stream)) return e;
-    if (weights == PSQ_Q8_E5M2)
-        return psq_gemm_fp8_e5m2w(q, K, sx, (const uint8_t *)w, ldw, w_scale, w_scale_per_row, bias, bias_dtype, y,
-                                  x_dtype, ldy, M, N, K, stream);
-    return psq_gemm_fp8_act(q, K, sx, (const uint8_t *)w, ldw, w_scale, w_scale_per_row, bias, bias_dtype, activation, y,
-                            x_dtype, ldy, M, N, K, stream);
+    const bool i8 = weights == PSQ_Q8_I8;
+    if (int e = i8 ? psq_quantize_rows_i8(x, x_dtype, M, K, ldx, rot_group, nullptr, (int8_t *)q, K, sx, stream)
+                   : psq_quantize_rows_fp8(x, x_dtype, M, K, ldx, 0, nullptr, q, K, sx, stream))
+        return e;
+    const int out = !y_f32 ? x_dtype : x_dtype == PSQ_BF16 ? Q8_WIDE_BF16 : Q8_WIDE_F16;
+    Q8Epi ep{sx, w_scale, i8 || w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_f32 ? 4 : 2)};
+    return run(i8 ? Q8_I8 : weights == PSQ_Q8_E4M3 ? Q8_E4M3 : Q8_E5M2W, out, activation,
+               {q, K, (const uint8_t *)w, ldw, M, N, K, ep, (hipStream_t)stream, name});
 }
 
 }  // extern "C"

@@ -31,12 +31,16 @@ struct Q8Args {
 // Operand kinds: int8 x int8, e4m3 x e4m3, e4m3 activations x e5m2 weights.
 enum { Q8_I8 = 0, Q8_E4M3 = 1, Q8_E5M2W = 2 };
 
+// Output types of the tiles: enum psq_dtype, 3 = int32 (256 x 256 int8 tiles only), and the bf16 / f16
+// outputs stored as fp32 (no activation; int8 and e4m3 weights).
+enum { Q8_OUT_I32 = 3, Q8_WIDE_BF16 = 4, Q8_WIDE_F16 = 5 };
+
 // Runs the problem on the small tiles (gemm_q8_small.hip) when they are the faster ones: true and its
 // status, or false and nothing launched.
 bool q8_small(int kind, int out, int act, const Q8Args &x, int &status);
 
-// The large tiles: 256 x 256 (every output and activation of its kind; out 3 = int32, int8 only), and
-// 256 x width, width 224, 192 or 160 (bf16 / f16 outputs, no gate).
+// The large tiles: 256 x 256 (every output and activation of its kind), and 256 x width, width 224, 192
+// or 160 (bf16 / f16 outputs, also stored as fp32; no gate).
 int q8_square_i8(int out, int act, const Q8Args &x);
 int q8_square_fp8(int kind, int out, int act, const Q8Args &x);
 int q8_width_i8(int width, int out, int act, const Q8Args &x);

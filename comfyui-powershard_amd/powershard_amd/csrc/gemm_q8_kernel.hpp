@@ -140,6 +140,16 @@ __device__ __forceinline__ uint32_t pack2g(float g0, float u0, float g1, float u
     return pack2<OUT>(silu(rg0) * ru0, silu(rg1) * ru1);
 }
 
+// Two packed words of 16-bit outputs as their four fp32 values.
+template <int OUT>
+__device__ __forceinline__ v4i widen2(int a, int b)
+{
+    if constexpr (OUT == OUT_BF16) return v4i{a << 16, (int)(a & 0xffff0000u), b << 16, (int)(b & 0xffff0000u)};
+    else
+        return v4i{__float_as_int(f16_to_f32((uint32_t)a & 0xffffu)), __float_as_int(f16_to_f32((uint32_t)a >> 16)),
+                   __float_as_int(f16_to_f32((uint32_t)b & 0xffffu)), __float_as_int(f16_to_f32((uint32_t)b >> 16))};
+}
+
 // One output element (the slow path of partial tiles and unaligned outputs).
 template <int OUT>
 __device__ __forceinline__ void store1(void *p, int c, float v)
@@ -226,7 +236,8 @@ __device__ __forceinline__ void tile_coords(int v, int nbm, int nbn, int &m0, in
 // gives each lane one output row and, per 32 x 32 tile, four runs of 4 consecutive columns: the
 // epilogue converts the accumulators in registers and stores them directly.
 // WF: the fp8 weights' format (0: e4m3fn, 1: e5m2), the f8f6f4 MFMA's A-operand format code.
-template <bool FP8, int OUT, int ACT, int WF, class L>
+// WIDE: the 16-bit outputs are stored as fp32 (their values; y is fp32).
+template <bool FP8, int OUT, int ACT, int WF, class L, bool WIDE>
 __global__ void __launch_bounds__(NTHREADS, 1)
 gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__restrict__ W, int64_t ldw,
                int M, int N, int K, Q8Epi ep)
@@ -242,6 +253,7 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
     constexpr int LA = L::LA, LW = L::LW, LPS = L::LPS, P = L::P, SCALE_WORDS = L::SCALE_WORDS;
     constexpr int STAGE_A = L::STAGE_A, STAGE_W = L::STAGE_W;
     constexpr bool MASKN = !FP8 || BN < 256;
+    static_assert(!WIDE || (ACT == ACT_NONE && (OUT == OUT_BF16 || OUT == OUT_F16)));
     static_assert(!GATED || (L::WGM == 2 && TN == 4));
 
     // wave-uniform values in scalar registers: the LDS destination of every global->LDS load (M0)
@@ -425,7 +437,7 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
     //   y = round_out(fmaf((float)acc, a_scale[m] * w_scale[n], bias[n]))
     auto epilogue = [&](int m0, int n0, int buf) {
         const uint32_t *sc = scale_lds + buf * SCALE_WORDS;
-        constexpr int esz = OUT == OUT_F32 || OUT == OUT_I32 ? 4 : 2;
+        constexpr int esz = WIDE || OUT == OUT_F32 || OUT == OUT_I32 ? 4 : 2;
         const int nl0 = wn * WAVE_N + 4 * (lane >> 5);
         uint8_t *rowp[TM];
         bool live[TM];
@@ -670,20 +682,29 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
                             val[q] = *(const v4i *)(eb + row * 128 + ((ch ^ chunk_xor(row)) << 4));
                         }
                         const int mb = m0 + wm * WAVE_M + 32 * i;   // first row of the block
-                        const int64_t ubase = ((int64_t)mb * ep.ldy + nb) * 2;
+                        const int64_t ubase = ((int64_t)mb * ep.ldy + nb) * esz;
+                        auto put = [&](const v4i &v, uint32_t loff) {
+                            v4i *dst = (v4i *)((uint8_t *)ep.y + ubase + loff);
+                            if constexpr (WIDE) {
+                                __builtin_nontemporal_store(widen2<OUT>(v[0], v[1]), dst);
+                                __builtin_nontemporal_store(widen2<OUT>(v[2], v[3]), dst + 1);
+                            } else {
+                                __builtin_nontemporal_store(v, dst);
+                            }
+                        };
                         if (mb + 32 <= M && (!MASKN || nb + 32 * NJ <= N)) {
 #pragma unroll
                             for (int q = 0; q < NST; q++) {
-                                const uint32_t loff = (uint32_t)(((RPS * q + (lane >> SH)) * ep.ldy + 8 * (lane & (CPR - 1))) * 2);
-                                __builtin_nontemporal_store(val[q], (v4i *)((uint8_t *)ep.y + ubase + loff));
+                                const uint32_t loff = (uint32_t)(((RPS * q + (lane >> SH)) * ep.ldy + 8 * (lane & (CPR - 1))) * esz);
+                                put(val[q], loff);
                             }
                         } else {
 #pragma unroll
                             for (int q = 0; q < NST; q++) {
                                 const int row = RPS * q + (lane >> SH), ch = lane & (CPR - 1);
                                 if (mb + row < M && (!MASKN || nb + 8 * ch + 8 <= N)) {
-                                    const uint32_t loff = (uint32_t)((row * ep.ldy + 8 * ch) * 2);
-                                    __builtin_nontemporal_store(val[q], (v4i *)((uint8_t *)ep.y + ubase + loff));
+                                    const uint32_t loff = (uint32_t)((row * ep.ldy + 8 * ch) * esz);
+                                    put(val[q], loff);
                                 }
                             }
                         }
@@ -693,7 +714,7 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
                 return;
             }
         }
-        if (ep.vec && n0 + BN <= N) {
+        if (!WIDE && ep.vec && n0 + BN <= N) {
             // Full-width tile, aligned rows.  Lanes l and l + 32 hold the same row: for column
             // groups g = 2p and 2p + 1 lane l has columns 16p + {0-3, 8-11} and lane l + 32 has
             // 16p + {4-7, 12-15}.  One v_permlane32_swap per word gives lane l columns 16p + 0-7
@@ -769,6 +790,7 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
                         for (int c = 0; c < 4; c++) {
                             if (!live[i] || c >= n_left0 - nc) continue;
                             if constexpr (OUT == OUT_I32) ((int32_t *)p)[c] = raw(i, j, 4 * g + c);
+                            else if constexpr (WIDE) ((float *)p)[c] = half_to_f32<OUT>(f32_to_half<OUT>(value(i, j, 4 * g + c, ws[c], bs[c])));
                             else store1<OUT>(p, c, act1<OUT, ACT>(value(i, j, 4 * g + c, ws[c], bs[c])));
                         }
                     }
@@ -960,10 +982,10 @@ gemm_q8_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__rest
     wait_vmcnt<0>();
 }
 
-template <bool FP8, int OUT, int ACT, int WF, class L>
+template <bool FP8, int OUT, int ACT, int WF, class L, bool WIDE = false>
 int launch_layout(const Q8Args &x)
 {
-    auto kern = gemm_q8_kernel<FP8, OUT, ACT, WF, L>;
+    auto kern = gemm_q8_kernel<FP8, OUT, ACT, WF, L, WIDE>;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return set_error(PSQ_E_DEVICE, "%s: no device", x.name);
     static bool attr_set[64] = {};   // per device; the attribute is idempotent
@@ -1005,13 +1027,15 @@ int launch_square(int out, int act, const Q8Args &x)
     case OUT_BF16: return launch_layout<FP8, OUT_BF16, ACT_NONE, 0, L>(x);
     case OUT_F16: return launch_layout<FP8, OUT_F16, ACT_NONE, 0, L>(x);
     case OUT_F32: return launch_layout<FP8, OUT_F32, ACT_NONE, 0, L>(x);
+    case Q8_WIDE_BF16: return launch_layout<FP8, OUT_BF16, ACT_NONE, 0, L, true>(x);
+    case Q8_WIDE_F16: return launch_layout<FP8, OUT_F16, ACT_NONE, 0, L, true>(x);
     default:
         if constexpr (!FP8) return launch_layout<FP8, OUT_I32, ACT_NONE, 0, L>(x);
         else return set_error(PSQ_E_ARG, "%s: bad output type", x.name);
     }
 }
 
-// 16-bit outputs of one narrower layout.
+// 16-bit outputs (as they are, or stored as fp32) of one narrower layout.
 template <bool FP8, int WF, class L>
 int launch_16bit(int out, int act, const Q8Args &x)
 {
@@ -1020,6 +1044,10 @@ int launch_16bit(int out, int act, const Q8Args &x)
             return out == OUT_BF16 ? launch_layout<FP8, OUT_BF16, ACT_GELU_TANH, WF, L>(x)
                                    : launch_layout<FP8, OUT_F16, ACT_GELU_TANH, WF, L>(x);
         else return set_error(PSQ_E_ARG, "%s: no activation for these weights", x.name);
+    }
+    if constexpr (WF == 0) {
+        if (out == Q8_WIDE_BF16) return launch_layout<FP8, OUT_BF16, ACT_NONE, WF, L, true>(x);
+        if (out == Q8_WIDE_F16) return launch_layout<FP8, OUT_F16, ACT_NONE, WF, L, true>(x);
     }
     return out == OUT_BF16 ? launch_layout<FP8, OUT_BF16, ACT_NONE, WF, L>(x)
                            : launch_layout<FP8, OUT_F16, ACT_NONE, WF, L>(x);

@@ -300,8 +300,9 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
     }
 
     // lane: output row 16 i + (lane & 15) of the wave's rows, columns 4 (lane >> 4) + 0..3 of tile j
-    auto finish = [&](auto outc) {
+    auto finish = [&](auto outc, auto widec) {
         constexpr int OUT = decltype(outc)::value;
+        constexpr bool WIDE = decltype(widec)::value;   // the 16-bit output's value stored as fp32
 #pragma unroll
         for (int j = 0; j < TO; j++) {
             const int n = n0 + (cg * TO + j) * 16 + 4 * fs;
@@ -328,7 +329,7 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
                 for (int c = 0; c < 4; c++) {
                     v[c] = __builtin_fmaf((float)acc[i][j][c], as * ws[0][c], bs[0][c]);
                     if constexpr (OUT == PSQ_BF16 || OUT == PSQ_F16) {
-                        if (act != ACT_NONE) v[c] = half_to_f32<OUT>(f32_to_half<OUT>(v[c]));
+                        if (WIDE || act != ACT_NONE) v[c] = half_to_f32<OUT>(f32_to_half<OUT>(v[c]));
                     }
                     if constexpr (GATE) {
                         float u = __builtin_fmaf((float)acc[i][j + TO][c], as * ws[NG - 1][c], bs[NG - 1][c]);
@@ -339,7 +340,7 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
                     }
                 }
                 const int64_t o = (int64_t)m * ep.ldy + n;
-                if constexpr (OUT == PSQ_F32) {
+                if constexpr (OUT == PSQ_F32 || WIDE) {
                     float *p = (float *)ep.y + o;
                     if (ep.vec && n + 4 <= NO) *(v4f *)p = v4f{v[0], v[1], v[2], v[3]};
                     else
@@ -360,9 +361,15 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
             }
         }
     };
-    if (out == PSQ_BF16) finish(std::integral_constant<int, PSQ_BF16>{});
-    else if (out == PSQ_F16) finish(std::integral_constant<int, PSQ_F16>{});
-    else finish(std::integral_constant<int, PSQ_F32>{});
+    using BF = std::integral_constant<int, PSQ_BF16>;
+    using HF = std::integral_constant<int, PSQ_F16>;
+    if (out == PSQ_BF16) finish(BF{}, std::false_type{});
+    else if (out == PSQ_F16) finish(HF{}, std::false_type{});
+    else if (out == PSQ_F32) finish(std::integral_constant<int, PSQ_F32>{}, std::false_type{});
+    else if constexpr (!GATE && KIND != 2) {
+        if (out == Q8_WIDE_BF16) finish(BF{}, std::true_type{});
+        else finish(HF{}, std::true_type{});
+    }
 }
 
 template <int KIND, int NW, int TM, int TN, int NRG, int NCG, int RA, int BUDGET, bool PIPE, bool GATE>

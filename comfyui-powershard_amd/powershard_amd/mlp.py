@@ -46,6 +46,20 @@ def silu_gate_linear(linear, rows):
     return F.silu(gate.float()) * up.float()
 
 
+def _down(fc2, hidden, rows):
+    """rows = fc2(hidden), in rows' dtype.  A plain QuantLinear whose output nothing else looks at
+    (no forward hook, no replaced forward) writes the rows from its GEMM's epilogue, widened to fp32
+    there where they are fp32; at 32760 x 5120 that replaces 154 us of conversion and 146 us of copy."""
+    if (type(fc2) is QuantLinear and "forward" not in fc2.__dict__ and not fc2._forward_hooks
+            and not torch.nn.modules.module._global_forward_hooks):
+        out = fc2(hidden, into=rows)
+        if out is rows:
+            return
+    else:
+        out = fc2(hidden)
+    rows.copy_(out)   # one pass, the conversion included
+
+
 def _chunk_step(n, chunk_tokens):
     if chunk_tokens is not None and int(chunk_tokens) <= 0:
         raise ValueError("chunk_tokens must be positive")
@@ -70,7 +84,7 @@ def gated_mlp(fc1, fc2, x, chunk_tokens=None, prepare_budget=None):
         for a in range(0, n, step):
             b = min(a + step, n)
             activation = silu_gate_linear(fc1, rows[a:b])
-            result[a:b] = fc2(activation)
+            _down(fc2, activation, result[a:b])
             del activation
     return result.reshape(shape[:-1] + (fc2.out_features,))
 
@@ -92,6 +106,6 @@ def chunked_mlp(fc1, fc2, x, chunk_tokens=None, prepare_budget=None):
         for a in range(0, n, step):
             b = min(a + step, n)
             hidden = gelu_linear(fc1, rows[a:b])
-            result[a:b] = fc2(hidden).float()
+            _down(fc2, hidden, result[a:b])
             del hidden
     return result.reshape(shape[:-1] + (fc2.out_features,))

@@ -316,23 +316,26 @@ def gemm_w8a16(x, wq, w_scale, bias=None, out_dtype=None):
 # host bounds: an int8 forward of one row 39 -> 17.8 us of host time, int4 28 -> 13.5 us.  The
 # arguments are as the general ops check them (QuantLinear._direct); None when the library refuses,
 # and the caller's general path then reports why.
-def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, act):
-    """x [..., K] contiguous bf16/f16; w, w_scale: device addresses.  [..., N] (gate: N / 2)."""
+def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, act, into=None):
+    """x [..., K] contiguous bf16/f16; w, w_scale: device addresses.  [..., N] (gate: N / 2) of x's
+    dtype; into: [M, N] rows of x's dtype or fp32 (the same values) that take the result."""
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
-    y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device)
+    y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device) if into is None else into
     scratch = torch.empty(((M * K + 15) & -16) + 4 * M, dtype=torch.uint8, device=x.device)
     status = lib.psq_linear_q8(weights, x.data_ptr(), dt, K, rot_group, w, K, w_scale, per_row,
-                               None if bias is None else bias.data_ptr(), dt, act, y.data_ptr(), cols, M, N, K,
-                               scratch.data_ptr(), _raw_stream(x.device.index))
+                               None if bias is None else bias.data_ptr(), dt, act, y.data_ptr(),
+                               int(y.dtype is torch.float32), cols, M, N, K, scratch.data_ptr(),
+                               _raw_stream(x.device.index))
     return None if status else y
 
 
-def linear_w4a16_direct(x, M, K, wq, w_scale, w_zero, group_size, N, bias):
-    """x [..., K] contiguous bf16/f16; wq, w_scale, w_zero: device addresses.  [..., N]."""
+def linear_w4a16_direct(x, M, K, wq, w_scale, w_zero, group_size, N, bias, into=None):
+    """x [..., K] contiguous bf16/f16; wq, w_scale, w_zero: device addresses.  [..., N]; into: [M, N]
+    rows of x's dtype that take the result."""
     lib, dt, stream = _native.lib(), _DT[x.dtype], _raw_stream(x.device.index)
     ws, nb = _workspace(x.device, stream or None, lib.psq_gemm_wonly_workspace_bytes(_native.W_UINT4, K, M, N, K, group_size))
-    y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+    y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device) if into is None else into
     status = lib.psq_gemm_w4a16_ws(x.data_ptr(), dt, K, wq, w_scale, w_zero, group_size,
                                    None if bias is None else bias.data_ptr(), dt, y.data_ptr(), dt, N, M, N, K,
                                    None if ws is None else ws.data_ptr(), nb, stream)

@@ -267,8 +267,11 @@ class QuantLinear(nn.Module):
     def extra_repr(self):
         return f"{self.in_features}, {self.out_features}, format={self._ps_qplan.fmt}, native={self._ps_native}"
 
-    def forward(self, x):
-        return self._forward(x, None)
+    def forward(self, x, into=None):
+        """self(x).  into (an MLP's result rows, [x rows, out_features]): memory that the native
+        kernels may write the output to, in its dtype; the caller copies when another tensor comes
+        back."""
+        return self._forward(x, None, into)
 
     def forward_act(self, x, activation="gelu_tanh"):
         """act(self(x)) with the activation fused into the native GEMM's epilogue.
@@ -329,7 +332,7 @@ class QuantLinear(nn.Module):
             tracker.observe(self._ps_finite_slot, out)
         return out
 
-    def _direct(self, x, activation):
+    def _direct(self, x, activation, into=None):
         """The native forward in one library call, or None where anything has to be converted,
         copied, shared, tracked, timed or refused: the general path below takes those (and reports
         what the library refuses).  Same kernels, same values."""
@@ -364,7 +367,9 @@ class QuantLinear(nn.Module):
             if (activation is not None or name != "zero" or sdtype is not torch.float16 or zdtype is not torch.float16
                     or K % group or s_bytes != 2 * N * (K // group) or z_bytes != s_bytes):
                 return None
-            return ops.linear_w4a16_direct(x, M, K, base + q_at, base + s_at, base + z_at, group, N, bias)
+            if into is not None and (into.dtype is not dtype or not _takes(into, device, M, N)):
+                into = None
+            return ops.linear_w4a16_direct(x, M, K, base + q_at, base + s_at, base + z_at, group, N, bias, into)
         weights, count, rot = _Q8_WEIGHTS.get(code), s_bytes // 4, 0
         if (weights is None or sdtype is not torch.float32 or (activation is not None and weights == 2)
                 or (activation == "silu_gate" and N % 128)):
@@ -376,12 +381,15 @@ class QuantLinear(nn.Module):
                 rot = plan.fields["convrot_groupsize"]
         elif layout is not qtm.Float8ScaledLayout or not weights or (count != N and count != 1):
             return None
+        if into is not None and ((into.dtype is not dtype and (into.dtype is not torch.float32 or weights == 2))
+                                 or not _takes(into, device, M, N)):
+            into = None
         return ops.linear_q8_direct(x, M, K, weights, base + q_at, base + s_at, int(count > 1), rot, N, bias,
-                                    ops.ACTIVATIONS[activation])
+                                    ops.ACTIVATIONS[activation], into)
 
-    def _forward(self, x, activation):
+    def _forward(self, x, activation, into=None):
         try:
-            out = self._direct(x, activation)
+            out = self._direct(x, activation, into)
         except torch.cuda.OutOfMemoryError:
             raise
         except NATIVE_FAILURES:   # e.g. a tensor without storage (vmap): the general path's policy applies
@@ -401,6 +409,12 @@ class QuantLinear(nn.Module):
         if activation is not None and not applied:
             out = apply_activation(out, activation)
         return self._deliver(out, x)
+
+
+def _takes(into, device, M, N):
+    """Whether plain rows `into` can take an [M, N] output as they are."""
+    return (type(into) is torch.Tensor and into.device == device and into.shape == (M, N) and into.is_contiguous()
+            and not into.requires_grad)
 
 
 # ------------------------------------------------------------------ shared activation quantization

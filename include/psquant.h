@@ -171,15 +171,17 @@ PSQ_API int psq_gemm_fp8_act(const uint8_t *a, int64_t lda, const float *a_scale
  *   weights     enum psq_q8_weights; e5m2 weights take no activation
  *   rot_group   int8 only, as in psq_quantize_rows_i8
  *   w [N, K], w_scale [N], or one value when w_scale_per_row is 0 (fp8)
- *   y           [M, N] (gate: [M, N / 2]) of x_dtype
+ *   y           [M, N] (gate: [M, N / 2]) of x_dtype; y_f32: fp32 holding the values rounded to x_dtype
+ *               (the Wan FFN's fc2(hidden).float(), powershard/wan_model.py:627; no activation, not for
+ *               e5m2 weights)
  *   scratch     16-byte aligned, psq_linear_q8_scratch_bytes(M, K) bytes: the codes, then the row scales.
  * The checks and the results of the separate calls. */
 enum psq_q8_weights { PSQ_Q8_I8 = 0, PSQ_Q8_E4M3 = 1, PSQ_Q8_E5M2 = 2 };
 PSQ_API int64_t psq_linear_q8_scratch_bytes(int64_t M, int64_t K);
 PSQ_API int psq_linear_q8(int weights, const void *x, int x_dtype, int64_t ldx, int rot_group, const void *w,
                   int64_t ldw, const float *w_scale, int w_scale_per_row, const void *bias, int bias_dtype,
-                  int activation, void *y, int64_t ldy, int64_t M, int64_t N, int64_t K, void *scratch,
-                  void *stream);
+                  int activation, void *y, int y_f32, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                  void *scratch, void *stream);
 
 /* W4A16: uint4 asymmetric group weights dequantized in registers,
  * w = round_bf16((float(q) - float(zero)) * float(scale)), multiplied on bf16 MFMA with

@@ -41,3 +41,23 @@ def test_width_matches_square_tiles(gpu, M, N, K, kind):
             assert torch.equal(y.cpu(), oracle.epilogue_i32(ops.gemm_i8_i32(a, w).cpu(), sa, sw, b, out_dtype=dt))
         if kind != "e5m2":
             assert_gelu_of(call(out_dtype=dt, activation="gelu_tanh"), y, f"{kind} {M}x{N}x{K} {dt}")
+
+
+# and: the 256 x 256 tiles, small tiles, outputs whose rows are not 16-byte aligned
+@pytest.mark.parametrize("M,N,K", SHAPES + [(2047, 7004, 128), (3000, 5000, 256), (3, 1000, 384), (100, 4999, 128),
+                                            (2000, 1500, 256), (1024, 8000, 128)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_fp32_rows_of_the_rounded_output(gpu, M, N, K, kind):
+    """psq_linear_q8's fp32 output holds the 16-bit output's values, bit for bit."""
+    from powershard_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(M + N)
+    w = codes(N, K, 5, torch.int8 if kind == 0 else torch.float8_e4m3fn, gpu, 0)
+    sw = torch.rand(N, generator=g, device=gpu) * 1e-2
+    for dt in (torch.bfloat16, torch.float16):
+        x = torch.randn(M, K, generator=g, device=gpu).to(dt)
+        b = torch.randn(N, generator=g, device=gpu).to(dt) if dt == torch.bfloat16 else None
+        call = lambda into: ops.linear_q8_direct(x, M, K, kind, w.data_ptr(), sw.data_ptr(), 1, 0, N, b, 0, into)
+        y = call(None)
+        wide, same = (torch.full((M, N), 7.0, dtype=t, device=gpu) for t in (torch.float32, dt))
+        assert call(wide) is wide and torch.equal(wide, y.float())
+        assert call(same) is same and torch.equal(same, y)
