@@ -40,6 +40,31 @@ struct WArgs {
     int sk = 0;
     float *part = nullptr;      // [2 sk][BM][256] fp32: the first and the last partial of each workgroup
     uint32_t *cnt = nullptr;    // [tiles] finished workgroups per tile: zero at launch, left zero
+    // int8: *flag = ticket when an output is NaN or +-Inf (null: not checked)
+    unsigned long long *flag = nullptr;
+    unsigned long long ticket = 0;
+};
+
+// Collects whether any stored output is NaN or +-Inf: the exponent of every element, plus its lowest
+// bit, carries into bits 15 / 31 when it is all ones.  Three VALU ops per two 16-bit outputs beside the
+// store, where a pass over the finished output cost 5.8 us at 1024 x 5120 and a launch.
+struct Finite {
+    uint32_t bad = 0;
+    __device__ __forceinline__ void half2(uint32_t w, int dt)
+    {
+        const uint32_t e = dt == PSQ_BF16 ? 0x7f807f80u : 0x7c007c00u, lsb = dt == PSQ_BF16 ? 0x00800080u : 0x04000400u;
+        bad |= (w & e) + lsb;
+    }
+    __device__ __forceinline__ void value(float v, int dt)   // one output as store_elem writes it
+    {
+        if (dt == PSQ_F32) bad |= ((__float_as_uint(v) & 0x7f800000u) + 0x00800000u) & 0x80000000u;
+        else half2(dt == PSQ_BF16 ? f32_to_bf16(v) : f32_to_f16(v), dt);
+    }
+    __device__ __forceinline__ void report(const WArgs &wa) const
+    {
+        // a plain store (the flag may be host memory): tickets only grow along the stream
+        if (wa.flag && (bad & 0x80008000u)) __hip_atomic_store(wa.flag, wa.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 };
 
 template <int XDT>
@@ -233,6 +258,7 @@ gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int
 #pragma unroll
         for (int v = 0; v < 4; v++) red[wave][mt][4 * h + v][nr] = acc[mt][v];
     __syncthreads();
+    Finite fin;
 #pragma unroll
     for (int o = tid; o < MT * 256; o += NTHREADS) {
         const int mt = o >> 8, ml = (o >> 4) & 15, nl = o & 15;
@@ -241,8 +267,11 @@ gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int
         const float sum = ((red[0][mt][nl][ml] + red[1][mt][nl][ml]) + red[2][mt][nl][ml]) + red[3][mt][nl][ml];
         const float cs = (WK == W_INT8) ? wa.scale32[nn] : 1.0f;
         const float bb = wa.bias ? load_elem(wa.bias, nn, wa.bias_dtype) : 0.0f;
-        store_elem(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, __builtin_fmaf(sum, cs, bb));
+        const float v = __builtin_fmaf(sum, cs, bb);
+        if constexpr (WK == W_INT8) fin.value(v, wa.y_dtype);
+        store_elem(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
     }
+    if constexpr (WK == W_INT8) fin.report(wa);
 }
 
 // ------------------------------------------------------------------ tiled kernel (M > 64)
@@ -696,6 +725,7 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
         auto value = [&](int i, int j, int r, float c, float b) {
             return __builtin_fmaf(__int_as_float(agpr_read(acc[i][j][r])), c, b);
         };
+        Finite fin;
         const bool fast = wa.y_dtype != PSQ_F32 && n0 + BN <= N && ((uintptr_t)wa.y & 15) == 0 && (wa.ldy * 2) % 16 == 0;
         if (fast) {
             // lanes l and l + 32 hold the same row: one v_permlane32_swap per word gives lane l columns
@@ -729,7 +759,16 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                             hi[d] = sw[1];
                         }
                         uint8_t *p = rowp[i] + (nc + 4 * h) * 2;
-                        if (live[i]) *(v4i *)p = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
+                        if (live[i]) {
+                            *(v4i *)p = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
+                            if constexpr (WK == W_INT8) {
+#pragma unroll
+                                for (int d = 0; d < 2; d++) {
+                                    fin.half2(lo[d], wa.y_dtype);
+                                    fin.half2(hi[d], wa.y_dtype);
+                                }
+                            }
+                        }
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -745,13 +784,17 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                         static_for<4>([&](auto cc) {
                             constexpr int c = decltype(cc)::value;
                             const float v = value(i, j, 4 * g + c, cs[c], bs[c]);
-                            if (live[i] && c < n_left0 - nc) store_elem(rowp[i], nc + c, wa.y_dtype, v);
+                            if (live[i] && c < n_left0 - nc) {
+                                store_elem(rowp[i], nc + c, wa.y_dtype, v);
+                                if constexpr (WK == W_INT8) fin.value(v, wa.y_dtype);
+                            }
                         });
                     });
                     __builtin_amdgcn_sched_barrier(0);
                 });
             });
         }
+        if constexpr (WK == W_INT8) fin.report(wa);
     }
 }
 
@@ -2004,13 +2047,16 @@ int gemm_w4a16(const void *x, int x_dtype, int64_t ldx, const uint8_t *wq, const
 
 int gemm_w8a16(const void *x, int x_dtype, int64_t ldx, const int8_t *wq, const float *w_scale, const void *bias,
                int bias_dtype, void *y, int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, void *workspace,
-               int64_t ws_bytes, void *stream, const char *name)
+               int64_t ws_bytes, void *stream, const char *name, unsigned long long *flag = nullptr,
+               unsigned long long ticket = 0)
 {
     if (int e = check_common(name, x, x_dtype, ldx, wq, y, y_dtype, ldy, bias, bias_dtype, M, N, K)) return e;
     if (M == 0 || N == 0) return PSQ_OK;
     if (!w_scale) return set_error(PSQ_E_ARG, "%s: null scale", name);
     if (int e = require_device()) return e;
     WArgs wa{(const uint8_t *)wq, nullptr, nullptr, w_scale, 0, bias, bias_dtype, y, y_dtype, ldy};
+    wa.flag = flag;
+    wa.ticket = ticket;
     return launch<W_INT8>(x, x_dtype, ldx, M, N, K, wa, workspace, ws_bytes, (hipStream_t)stream, name);
 }
 
@@ -2100,6 +2146,27 @@ int psq_gemm_w4a16_noalloc(const void *x, int x_dtype, int64_t ldx, const uint8_
     if (int e = scratch_on_device(&ptr)) return e;
     return gemm_w4a16(x, x_dtype, ldx, wq, w_scale, w_zero, group_size, bias, bias_dtype, y, y_dtype, ldy, M, N, K,
                       ptr, kMaxWsBytes, stream, "gemm_w4a16_noalloc");
+}
+
+int psq_linear_w8a16(const void *x, int x_dtype, int64_t ldx, int rot_group, const int8_t *wq, const float *w_scale,
+                     const void *bias, int bias_dtype, void *y, int64_t ldy, int64_t M, int64_t N, int64_t K,
+                     void *rotated, void *workspace, int64_t workspace_bytes, unsigned long long *flag,
+                     unsigned long long ticket, void *stream)
+{
+    using namespace psq;
+    const char *name = "linear_w8a16";
+    if (!flag || ((uintptr_t)flag & 7) || !ticket) return set_error(PSQ_E_ARG, "%s: no flag or ticket", name);
+    const void *rows = x;
+    if (rot_group) {
+        // refuse before the rotation runs what the GEMM would refuse
+        if (int e = check_common(name, rotated, x_dtype, K, wq, y, x_dtype, ldy, bias, bias_dtype, M, N, K)) return e;
+        if (M == 0 || N == 0) return PSQ_OK;
+        if (int e = psq_rotate_rows(x, x_dtype, M, K, ldx, rot_group, rotated, x_dtype, K, stream)) return e;
+        rows = rotated;
+        ldx = K;
+    }
+    return gemm_w8a16(rows, x_dtype, ldx, wq, w_scale, bias, bias_dtype, y, x_dtype, ldy, M, N, K, workspace,
+                      workspace_bytes, stream, name, flag, ticket);
 }
 
 int64_t psq_gemm_wonly_workspace_bytes(int weight_kind, int64_t ldx, int64_t M, int64_t N, int64_t K, int group_size)

@@ -75,7 +75,9 @@ class Int8Linear(nn.Module):
             # defers to one read per forward (fp16_safe.py FiniteTracker.finish): the tracker must
             # not see an overflow the tile path would not have produced.
             if out is not None:
-                finite = not ops.any_nonfinite(out)
+                out, finite = out
+                if finite is None:
+                    finite = not ops.any_nonfinite(out)
                 if not finite:
                     out = None
         if out is None:
@@ -103,8 +105,9 @@ class Int8Linear(nn.Module):
         return getattr(self, "_ps_safe", False) or self.weight.device.type != "cuda" or not getattr(self, "_ps_native", True)
 
     def _native_forward(self, x, check):
-        """fp16 x [..., K] -> fp16 [..., N] on the gfx950 kernels, or None (and the tile path from
-        then on) when the kernels do not take the shape.  A missing library raises (as on the tile
+        """fp16 x [..., K] -> (fp16 [..., N], whether it is finite, None where that is still to be
+        checked) on the gfx950 kernels, or None (and the tile path from then on) when the kernels do
+        not take the shape.  A missing library raises (as on the tile
         path, whose GPU dequantization is a kernel too).  The dequantized weight's fp16 range check
         of the tile path (dequantize_rows) is kept as a bound, once: every element of (q s) H^T is
         at most sqrt(g) max|q s| in magnitude."""
@@ -117,15 +120,24 @@ class Int8Linear(nn.Module):
                 self._ps_native = False
                 return None
             self._ps_range_ok = True
-        rows = x.reshape(-1, self.in_features).contiguous()
         bias = None if self.bias is None else self.bias.to(torch.float16)
+        weight, scale, rot = self.weight, self.weight_scale, self.group_size if self.convrot else 0
+        N, K = weight.shape
         try:
+            if (type(x) is torch.Tensor and x.numel() and x.shape[-1] == K == self.in_features and x.is_contiguous()
+                    and weight.dtype is torch.int8 and weight.is_contiguous() and weight.device == x.device
+                    and scale.dtype is torch.float32 and scale.is_contiguous() and scale.numel() == N
+                    and scale.device == x.device and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+                    and (bias is None or (bias.numel() == N and bias.is_contiguous() and bias.device == x.device))
+                    and ops.direct_available()):
+                return ops.linear_w8a16_direct(x, x.numel() // K, K, weight, scale, rot, N, bias)
+            rows = x.reshape(-1, self.in_features).contiguous()
             xr = ops.rotate_rows(rows, self.group_size) if self.convrot else rows
             y = ops.gemm_w8a16(xr, self.weight, self.weight_scale, bias, out_dtype=torch.float16)
         except RuntimeError:
             self._ps_native = False
             return None
-        return y.reshape(x.shape[:-1] + (self.out_features,))
+        return y.reshape(x.shape[:-1] + (self.out_features,)), None
 
 
 def install_int8(model, quant, rows):

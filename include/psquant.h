@@ -240,6 +240,17 @@ PSQ_API int psq_gemm_w8a16_ws(const void *x, int x_dtype, int64_t ldx, const int
                       int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, void *workspace,
                       int64_t workspace_bytes, void *stream);
 
+/* Int8Linear's forward (powershard/operations.py:96-132) in one call: psq_rotate_rows of x into
+ * `rotated` ([M, K] of x_dtype, 16-byte aligned; unused for rot_group 0), psq_gemm_w8a16_ws of the
+ * rows, output of x_dtype, and the output check of psq_flag_nonfinite in the GEMM's epilogue: *flag
+ * (device memory, or host memory that the device can write) becomes `ticket` when an output is NaN or
+ * +-Inf.  One flag per stream, tickets from 1 and increasing along it. */
+PSQ_API int psq_linear_w8a16(const void *x, int x_dtype, int64_t ldx, int rot_group, const int8_t *wq,
+                     const float *w_scale, const void *bias, int bias_dtype, void *y, int64_t ldy,
+                     int64_t M, int64_t N, int64_t K, void *rotated, void *workspace,
+                     int64_t workspace_bytes, unsigned long long *flag, unsigned long long ticket,
+                     void *stream);
+
 /* psq_gemm_w4a16_ws without the workspace argument: the split-K counters and partial tiles live in
  * a static device array of the library (64 MB + 64 KB on each GPU it runs on, held until the
  * process ends), so the call allocates nothing -- no hipMalloc, no hipFree, no allocating library
