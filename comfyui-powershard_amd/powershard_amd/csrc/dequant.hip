@@ -22,10 +22,24 @@ __device__ __forceinline__ void store16(void *out, int64_t base, const float (&v
     } else {
         uint32_t h[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) h[i] = f32_to_half<ODT>(v[2 * i]) | (f32_to_half<ODT>(v[2 * i + 1]) << 16);
+        for (int i = 0; i < 8; i++) h[i] = pack_half2<ODT>(v[2 * i], v[2 * i + 1]);
         v4i *o = (v4i *)((uint16_t *)out + base);
         o[0] = v4i{(int)h[0], (int)h[1], (int)h[2], (int)h[3]};
         o[1] = v4i{(int)h[4], (int)h[5], (int)h[6], (int)h[7]};
+    }
+}
+
+// Row n and first k of thread id's 16 values.  A 64-bit division is some 100 instructions, so sizes that
+// fit take it in 32 bits.
+__device__ __forceinline__ void row_of(int64_t id, int64_t N, int64_t per_row, int64_t &n, int64_t &k0)
+{
+    if (N * per_row <= 0x7fffffff) {
+        const uint32_t r = (uint32_t)id / (uint32_t)per_row;
+        n = r;
+        k0 = 16 * (int64_t)((uint32_t)id - r * (uint32_t)per_row);
+    } else {
+        n = id / per_row;
+        k0 = 16 * (id - n * per_row);
     }
 }
 
@@ -38,13 +52,14 @@ dequant_uint4_kernel(const uint8_t *__restrict__ wq, const uint16_t *__restrict_
     const int64_t per_row = K / 16;
     const int64_t id = (int64_t)blockIdx.x * NT + threadIdx.x;
     if (id >= N * per_row) return;
-    const int64_t n = id / per_row, k0 = (id % per_row) * 16;
+    int64_t n, k0;
+    row_of(id, N, per_row, n, k0);
     const v2i p = *(const v2i *)(wq + n * (K / 2) + k0 / 2);
     float v[16];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         // a group boundary can fall inside these 16 values only when gs < 16 (gs >= 16 enforced)
-        const int64_t gi = n * (K / gs) + (k0 + 8 * h) / gs;
+        const int64_t gi = n * ((uint32_t)K / (uint32_t)gs) + (uint32_t)(k0 + 8 * h) / (uint32_t)gs;
         const float s = f16_to_f32(sc[gi]), z = f16_to_f32(zp[gi]);
         const uint32_t w = (uint32_t)p[h];
 #pragma unroll
@@ -62,7 +77,8 @@ dequant_fp8_kernel(const uint8_t *__restrict__ q, const float *__restrict__ sc, 
     const int64_t per_row_t = K / 16;
     const int64_t id = (int64_t)blockIdx.x * NT + threadIdx.x;
     if (id >= N * per_row_t) return;
-    const int64_t n = id / per_row_t, k0 = (id % per_row_t) * 16;
+    int64_t n, k0;
+    row_of(id, N, per_row_t, n, k0);
     const v4i p = *(const v4i *)(q + n * K + k0);
     const float s = sc[per_row ? n : 0];
     float v[16];
@@ -75,52 +91,43 @@ dequant_fp8_kernel(const uint8_t *__restrict__ q, const float *__restrict__ sc, 
 }
 
 // int8 rows: one workgroup per row; thread t owns P chunks of 16 consecutive values, chunk c at
-// elements [(c T + t) 16, +16) (T = blockDim.x, a multiple of 64), so each wave covers 1024
+// elements [(c T + lane_chunk(t)) 16, +16) (T = blockDim.x, a multiple of 64), so each wave covers 1024
 // consecutive values per chunk and ConvRot groups (at most 1024, dividing K) never straddle waves.
-// The ConvRot inverse is the quantizer's transform (H is symmetric, so v @ H^T = 2^-k T(v)).
+// The ConvRot inverse is the quantizer's transform (H is symmetric, so v @ H^T = 2^-k T(v)), its lane
+// stages leaving their digits reversed: the thread's results belong to the chunk of lane
+// t ^ rev_lanes, the same values as the digit-ordered stages with fewer exchanges.
 // Lanes past K carry zeros through the cross-lane stages: their groups lie wholly past K.
+// The int8 rows and their scales are streamed; without the rotation the pass is HBM-bound, with it the
+// transform's VALU work shows: 13824 x 5120 to bf16 36.2 us (5.9 TB/s), with group 256 51.1 -> 39.7 us
+// (5.35 TB/s) against digit-ordered stages and a rounding written out in integer ops, group 1024 57.3 ->
+// 46.4 us.  The uint4 pass went 41.9 -> 36.4 us (packed rounding, 32-bit row division).
 template <int ODT, int ROTK, int P>
 __global__ void __launch_bounds__(1024)
 dequant_i8_rows_kernel(const int8_t *__restrict__ q, const float *__restrict__ sc, int64_t K, void *__restrict__ out)
 {
     const int64_t n = blockIdx.x;
-    const int t = threadIdx.x, T = blockDim.x;
+    const int t = threadIdx.x, T = blockDim.x, lc = lane_chunk<ROTK>(t);
     const float s = sc[n];
+    v4i p[P];
 #pragma unroll
     for (int c = 0; c < P; c++) {
-        const int64_t e0 = (int64_t)(c * T + t) * 16;
-        const bool active = e0 < K;
+        const int64_t e0 = (int64_t)(c * T + lc) * 16;
+        p[c] = v4i{0, 0, 0, 0};
+        if (e0 < K) p[c] = __builtin_nontemporal_load((const v4i *)(q + n * K + e0));
+    }
+#pragma unroll
+    for (int c = 0; c < P; c++) {
         float v[16];
-        v4i p = {0, 0, 0, 0};
-        if (active) p = *(const v4i *)(q + n * K + e0);
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = (float)(int8_t)(((uint32_t)p[i >> 2] >> (8 * (i & 3))) & 0xffu) * s;
-        if constexpr (ROTK >= 1) {
-#pragma unroll
-            for (int b = 0; b < 16; b += 4) radix4(v[b], v[b + 1], v[b + 2], v[b + 3]);
-        }
-        if constexpr (ROTK >= 2) {
-#pragma unroll
-            for (int a = 0; a < 4; a++) radix4(v[a], v[a + 4], v[a + 8], v[a + 12]);
-        }
-        if constexpr (ROTK >= 3) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = radix4_lanes<1>(v[j]);
-        }
-        if constexpr (ROTK >= 4) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = radix4_lanes<4>(v[j]);
-        }
-        if constexpr (ROTK >= 5) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = radix4_lanes<16>(v[j]);
-        }
+        for (int i = 0; i < 16; i++) v[i] = (float)(int8_t)(((uint32_t)p[c][i >> 2] >> (8 * (i & 3))) & 0xffu) * s;
+        rotate16<ROTK>(v);
         if constexpr (ROTK > 0) {
             const float post = __builtin_ldexpf(1.0f, -ROTK);
 #pragma unroll
             for (int j = 0; j < 16; j++) v[j] = v[j] * post;
         }
-        if (active) store16<ODT>(out, n * K + e0, v);
+        const int64_t e0 = (int64_t)(c * T + (lc ^ rev_lanes<ROTK>())) * 16;
+        if (e0 < K) store16<ODT>(out, n * K + e0, v);
     }
 }
 

@@ -177,7 +177,7 @@ __device__ __forceinline__ float dpp(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
-// value of lane ^ (m * L) for the three radix-4 partners at lane stride L in {1, 4}
+// value of lane ^ (m * L) for the three radix-4 partners at lane stride L
 template <int L, int M_>
 __device__ __forceinline__ float lane_xor(float v)
 {
@@ -185,10 +185,6 @@ __device__ __forceinline__ float lane_xor(float v)
         if constexpr (M_ == 1) return dpp<DPP_QUAD_XOR1>(v);
         else if constexpr (M_ == 2) return dpp<DPP_QUAD_XOR2>(v);
         else return dpp<DPP_QUAD_XOR3>(v);
-    } else if constexpr (L == 4) {
-        if constexpr (M_ == 1) return dpp<DPP_QUAD_XOR3>(dpp<DPP_ROW_HALF_MIRROR>(v));  // ^7 ^3 = ^4
-        else if constexpr (M_ == 2) return dpp<DPP_ROW_ROR8>(v);                          // ^8
-        else return dpp<DPP_QUAD_XOR3>(dpp<DPP_ROW_MIRROR>(v));                           // ^15 ^3 = ^12
     } else {
         return __shfl_xor(v, L * M_, 64);
     }
@@ -241,6 +237,47 @@ __device__ __forceinline__ float radix4_lanes_rev_sw4(float x)
     float t = x + dpp<DPP_ROW_ROR8>(x);
     float s = t + dpp<DPP_ROW_ROR4>(t);
     return __builtin_fmaf(-2.0f, x, s);
+}
+
+// Unnormalized transform of the 16 values of this thread (in-thread digits) and of the
+// cross-lane digits, for a group size of 4^ROTK.  Digits 2 and 3 (lane bits 0-1 and 2-3) come out
+// reversed (radix4_lanes_rev): the thread's 16 results belong to the chunk of thread t ^ rev_lanes.
+template <int ROTK>
+constexpr int rev_lanes() { return (ROTK >= 3 ? 3 : 0) | (ROTK >= 4 ? 12 : 0); }
+
+// Chunk (within its wave's 64) that lane t loads: lane bits 2 and 3 swapped when digit 3 lives on
+// them (see radix4_lanes_rev_sw4), so the chunk's digit-3 bit 0 sits on lane bit 3.  The wave's
+// loads and stores cover the same 2 KB and 1 KB as in lane order.
+template <int ROTK>
+__device__ __forceinline__ int lane_chunk(int t)
+{
+    if constexpr (ROTK >= 4) return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1);
+    else return t;
+}
+
+template <int ROTK>
+__device__ __forceinline__ void rotate16(float (&v)[16])
+{
+    if constexpr (ROTK >= 1) {
+#pragma unroll
+        for (int b = 0; b < 16; b += 4) radix4(v[b], v[b + 1], v[b + 2], v[b + 3]);
+    }
+    if constexpr (ROTK >= 2) {
+#pragma unroll
+        for (int a = 0; a < 4; a++) radix4(v[a], v[a + 4], v[a + 8], v[a + 12]);
+    }
+    if constexpr (ROTK >= 3) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = radix4_lanes_rev<1>(v[j]);
+    }
+    if constexpr (ROTK >= 4) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = radix4_lanes_rev_sw4(v[j]);
+    }
+    if constexpr (ROTK >= 5) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = radix4_lanes<16>(v[j]);
+    }
 }
 
 // ------------------------------------------------------------------ XCD-aware tile order

@@ -112,47 +112,6 @@ __device__ __forceinline__ uint32_t i8_codes4(float u0, float u1, float u2, floa
     return w;
 }
 
-// Unnormalized transform of the 16 values of this thread (in-thread digits) and of the
-// cross-lane digits, for a group size of 4^ROTK.  Digits 2 and 3 (lane bits 0-1 and 2-3) come out
-// reversed (radix4_lanes_rev): the thread's 16 results belong to the chunk of thread t ^ rev_lanes.
-template <int ROTK>
-constexpr int rev_lanes() { return (ROTK >= 3 ? 3 : 0) | (ROTK >= 4 ? 12 : 0); }
-
-// Chunk (within its wave's 64) that lane t loads: lane bits 2 and 3 swapped when digit 3 lives on
-// them (see radix4_lanes_rev_sw4), so the chunk's digit-3 bit 0 sits on lane bit 3.  The wave's
-// loads and stores cover the same 2 KB and 1 KB as in lane order.
-template <int ROTK>
-__device__ __forceinline__ int lane_chunk(int t)
-{
-    if constexpr (ROTK >= 4) return (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1);
-    else return t;
-}
-
-template <int ROTK>
-__device__ __forceinline__ void rotate16(float (&v)[16])
-{
-    if constexpr (ROTK >= 1) {
-#pragma unroll
-        for (int b = 0; b < 16; b += 4) radix4(v[b], v[b + 1], v[b + 2], v[b + 3]);
-    }
-    if constexpr (ROTK >= 2) {
-#pragma unroll
-        for (int a = 0; a < 4; a++) radix4(v[a], v[a + 4], v[a + 8], v[a + 12]);
-    }
-    if constexpr (ROTK >= 3) {
-#pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = radix4_lanes_rev<1>(v[j]);
-    }
-    if constexpr (ROTK >= 4) {
-#pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = radix4_lanes_rev_sw4(v[j]);
-    }
-    if constexpr (ROTK >= 5) {
-#pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = radix4_lanes<16>(v[j]);
-    }
-}
-
 // A workgroup quantizes R consecutive rows side by side (all their loads issued up front, one
 // shared barrier for the absmax reductions).  Thread t owns P chunks of 16 consecutive elements
 // of each row: chunk c = elements [(c T + lane_chunk(t)) 16, +16), T = blockDim.x (a multiple of
