@@ -1,6 +1,7 @@
 // gemm_q8.hip -- entry points of the W8A8 int8 and fp8 GEMMs: argument checks and the choice of tiles.
 // The kernels: gemm_q8_kernel.hpp (large tiles), gemm_q8_small.hip (small tiles, split K).
 #include "gemm_q8.hpp"
+#include "quantize.hpp"
 
 namespace psq {
 namespace {
@@ -186,23 +187,30 @@ int psq_linear_q8(int weights, const void *x, int x_dtype, int64_t ldx, int rot_
     if (weights != PSQ_Q8_I8 && rot_group) return set_error(PSQ_E_ARG, "%s: the rotation is int8's", name);
     if (x_dtype != PSQ_BF16 && x_dtype != PSQ_F16) return set_error(PSQ_E_ARG, "%s: activations must be bf16/f16", name);
     if (bias && !valid_dtype(bias_dtype)) return set_error(PSQ_E_ARG, "%s: bad dtype", name);
-    if (M > 0 && N > 0 && K > 0 && (!scratch || ((uintptr_t)scratch & 15)))
-        return set_error(PSQ_E_ARG, "%s: scratch must be 16-byte aligned", name);
-    // refuse before the quantizer runs what the GEMM would refuse
-    if (int e = check_shapes(name, scratch, K, w, ldw, M, N, K)) return e;
+    // refuse before the quantizer runs what the GEMM would refuse (its operand `a` is made here)
+    if (int e = check_shapes(name, w, K, w, ldw, M, N, K)) return e;
     if (int e = check_act(name, activation, N, ldw, K, ldy)) return e;
     if (M == 0 || N == 0) return PSQ_OK;
     if (!w_scale || !y) return set_error(PSQ_E_ARG, "%s: null scale or output", name);
     uint8_t *q = (uint8_t *)scratch;
     float *sx = (float *)(q + ((M * K + 15) & ~15LL));
     const bool i8 = weights == PSQ_Q8_I8;
+    const int kind = i8 ? Q8_I8 : weights == PSQ_Q8_E4M3 ? Q8_E4M3 : Q8_E5M2W;
+    Q8Epi ep{sx, w_scale, i8 || w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_f32 ? 4 : 2)};
+    const Q8Args args{q, K, (const uint8_t *)w, ldw, M, N, K, ep, (hipStream_t)stream, name};
+    // one or two rows: quantized by the GEMM itself (what the quantizer would refuse goes to it)
+    int rotk = 0;
+    if (q8_vec_fits(M, K, activation) && x && ((uintptr_t)x & 15) == 0 && ldx >= K && ldx % 8 == 0 &&
+        rot_log4(rot_group, K, rotk) == PSQ_OK) {
+        if (int e = require_device()) return e;
+        return q8_vec(kind, x, x_dtype, ldx, rotk, y_f32 ? 1 : 0, activation, args);
+    }
+    if (!scratch || ((uintptr_t)scratch & 15)) return set_error(PSQ_E_ARG, "%s: scratch must be 16-byte aligned", name);
     if (int e = i8 ? psq_quantize_rows_i8(x, x_dtype, M, K, ldx, rot_group, nullptr, (int8_t *)q, K, sx, stream)
                    : psq_quantize_rows_fp8(x, x_dtype, M, K, ldx, 0, nullptr, q, K, sx, stream))
         return e;
     const int out = !y_f32 ? x_dtype : x_dtype == PSQ_BF16 ? Q8_WIDE_BF16 : Q8_WIDE_F16;
-    Q8Epi ep{sx, w_scale, i8 || w_scale_per_row ? 1 : 0, bias, bias_dtype, y, ldy, vec_ok(y, ldy, y_f32 ? 4 : 2)};
-    return run(i8 ? Q8_I8 : weights == PSQ_Q8_E4M3 ? Q8_E4M3 : Q8_E5M2W, out, activation,
-               {q, K, (const uint8_t *)w, ldw, M, N, K, ep, (hipStream_t)stream, name});
+    return run(kind, out, activation, args);
 }
 
 }  // extern "C"

@@ -39,6 +39,11 @@ enum { Q8_OUT_I32 = 3, Q8_WIDE_BF16 = 4, Q8_WIDE_F16 = 5 };
 // status, or false and nothing launched.
 bool q8_small(int kind, int out, int act, const Q8Args &x, int &status);
 
+// Quantizes one or two rows x itself (gemm_q8_vec.hip) where q8_vec_fits: a checked call whose operand
+// `a` and row scales are not used.  wide: y is fp32.
+bool q8_vec_fits(int64_t M, int64_t K, int act);
+int q8_vec(int kind, const void *x, int x_dtype, int64_t ldx, int rotk, int wide, int act, const Q8Args &a);
+
 // The large tiles: 256 x 256 (every output and activation of its kind), and 256 x width, width 224, 192
 // or 160 (bf16 / f16 outputs, also stored as fp32; no gate).
 int q8_square_i8(int out, int act, const Q8Args &x);

@@ -312,8 +312,9 @@ def gemm_w8a16(x, wq, w_scale, bias=None, out_dtype=None):
 
 # ------------------------------------------------------- module forward in one call
 # The launches of a QuantLinear forward with nothing to convert: addresses and sizes straight to the
-# library, one scratch allocation, no tensor per stored component.  For the small calls, which the
-# host bounds: an int8 forward of one row 39 -> 17.8 us of host time, int4 28 -> 13.5 us.  The
+# library, at most one scratch allocation, no tensor per stored component.  For the small calls, which
+# the host bounds: an int8 or fp8 forward 39 -> 17.8 us of host time (one or two rows, quantized inside
+# the GEMM: 13.8 us), int4 28 -> 13.5 us.  The
 # arguments are as the general ops check them (QuantLinear._direct); None when the library refuses,
 # and the caller's general path then reports why.
 def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, act, into=None):
@@ -322,10 +323,13 @@ def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, 
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
     y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device) if into is None else into
-    scratch = torch.empty(((M * K + 15) & -16) + 4 * M, dtype=torch.uint8, device=x.device)
+    # (one or two rows are quantized inside the GEMM: no scratch, see psq_linear_q8)
+    scratch = None if M <= 2 and K <= 8192 and act != ACTIVATIONS["silu_gate"] else \
+        torch.empty(((M * K + 15) & -16) + 4 * M, dtype=torch.uint8, device=x.device)
     status = lib.psq_linear_q8(weights, x.data_ptr(), dt, K, rot_group, w, K, w_scale, per_row,
                                None if bias is None else bias.data_ptr(), dt, act, y.data_ptr(),
-                               int(y.dtype is torch.float32), cols, M, N, K, scratch.data_ptr(),
+                               int(y.dtype is torch.float32), cols, M, N, K,
+                               None if scratch is None else scratch.data_ptr(),
                                _raw_stream(x.device.index))
     return None if status else y
 

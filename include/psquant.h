@@ -175,6 +175,8 @@ PSQ_API int psq_gemm_fp8_act(const uint8_t *a, int64_t lda, const float *a_scale
  *               (the Wan FFN's fc2(hidden).float(), powershard/wan_model.py:627; no activation, not for
  *               e5m2 weights)
  *   scratch     16-byte aligned, psq_linear_q8_scratch_bytes(M, K) bytes: the codes, then the row scales.
+ *               One or two rows of at most 8192 elements without the gate are quantized inside the GEMM
+ *               and use none (NULL is accepted).
  * The checks and the results of the separate calls. */
 enum psq_q8_weights { PSQ_Q8_I8 = 0, PSQ_Q8_E4M3 = 1, PSQ_Q8_E5M2 = 2 };
 PSQ_API int64_t psq_linear_q8_scratch_bytes(int64_t M, int64_t K);
