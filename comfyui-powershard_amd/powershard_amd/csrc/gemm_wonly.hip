@@ -47,7 +47,7 @@ struct WArgs {
 
 // Collects whether any stored output is NaN or +-Inf: the exponent of every element, plus its lowest
 // bit, carries into bits 15 / 31 when it is all ones.  Three VALU ops per two 16-bit outputs beside the
-// store, where a pass over the finished output cost 5.8 us at 1024 x 5120 and a launch.
+// store (of a checked call), where a pass over the finished output cost 5.8 us at 1024 x 5120 and a launch.
 struct Finite {
     uint32_t bad = 0;
     __device__ __forceinline__ void half2(uint32_t w, int dt)
@@ -55,10 +55,17 @@ struct Finite {
         const uint32_t e = dt == PSQ_BF16 ? 0x7f807f80u : 0x7c007c00u, lsb = dt == PSQ_BF16 ? 0x00800080u : 0x04000400u;
         bad |= (w & e) + lsb;
     }
-    __device__ __forceinline__ void value(float v, int dt)   // one output as store_elem writes it
+    // one output, stored as store_elem does
+    __device__ __forceinline__ void store(void *p, int64_t i, int dt, float v)
     {
-        if (dt == PSQ_F32) bad |= ((__float_as_uint(v) & 0x7f800000u) + 0x00800000u) & 0x80000000u;
-        else half2(dt == PSQ_BF16 ? f32_to_bf16(v) : f32_to_f16(v), dt);
+        if (dt == PSQ_F32) {
+            ((float *)p)[i] = v;
+            bad |= ((__float_as_uint(v) & 0x7f800000u) + 0x00800000u) & 0x80000000u;
+        } else {
+            const uint32_t h = dt == PSQ_BF16 ? f32_to_bf16(v) : f32_to_f16(v);
+            ((uint16_t *)p)[i] = (uint16_t)h;
+            half2(h, dt);
+        }
     }
     __device__ __forceinline__ void report(const WArgs &wa) const
     {
@@ -268,8 +275,8 @@ gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int
         const float cs = (WK == W_INT8) ? wa.scale32[nn] : 1.0f;
         const float bb = wa.bias ? load_elem(wa.bias, nn, wa.bias_dtype) : 0.0f;
         const float v = __builtin_fmaf(sum, cs, bb);
-        if constexpr (WK == W_INT8) fin.value(v, wa.y_dtype);
-        store_elem(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
+        if (WK == W_INT8 && wa.flag) fin.store(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
+        else store_elem(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
     }
     if constexpr (WK == W_INT8) fin.report(wa);
 }
@@ -761,7 +768,7 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                         uint8_t *p = rowp[i] + (nc + 4 * h) * 2;
                         if (live[i]) {
                             *(v4i *)p = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
-                            if constexpr (WK == W_INT8) {
+                            if (WK == W_INT8 && wa.flag) {
 #pragma unroll
                                 for (int d = 0; d < 2; d++) {
                                     fin.half2(lo[d], wa.y_dtype);
@@ -785,8 +792,8 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                             constexpr int c = decltype(cc)::value;
                             const float v = value(i, j, 4 * g + c, cs[c], bs[c]);
                             if (live[i] && c < n_left0 - nc) {
-                                store_elem(rowp[i], nc + c, wa.y_dtype, v);
-                                if constexpr (WK == W_INT8) fin.value(v, wa.y_dtype);
+                                if (WK == W_INT8 && wa.flag) fin.store(rowp[i], nc + c, wa.y_dtype, v);
+                                else store_elem(rowp[i], nc + c, wa.y_dtype, v);
                             }
                         });
                     });

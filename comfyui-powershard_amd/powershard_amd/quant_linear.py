@@ -388,14 +388,15 @@ class QuantLinear(nn.Module):
                                     ops.ACTIVATIONS[activation], into)
 
     def _forward(self, x, activation, into=None):
-        try:
-            out = self._direct(x, activation, into)
-        except torch.cuda.OutOfMemoryError:
-            raise
-        except NATIVE_FAILURES:   # e.g. a tensor without storage (vmap): the general path's policy applies
-            out = None
-        if out is not None:
-            return out
+        if self._ps_native:
+            try:
+                out = self._direct(x, activation, into)
+            except torch.cuda.OutOfMemoryError:
+                raise
+            except NATIVE_FAILURES:   # e.g. a tensor without storage (vmap): the general path's policy applies
+                out = None
+            if out is not None:
+                return out
         dtype = self._dtype_for(x)
         qt, extras = unpack(self.qbytes, self._ps_qplan, dtype, with_extras=True)
         rows = x.reshape(-1, x.shape[-1]).to(dtype)
