@@ -69,7 +69,7 @@ struct Finite {
     }
     __device__ __forceinline__ void report(const WArgs &wa) const
     {
-        // a plain store (the flag may be host memory): tickets only grow along the stream
+        // a plain store (the flag may be host memory): the flag has one caller, whose tickets grow
         if (wa.flag && (bad & 0x80008000u)) __hip_atomic_store(wa.flag, wa.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 };

@@ -130,7 +130,9 @@ class Int8Linear(nn.Module):
                     and scale.device == x.device and (x.data_ptr() | weight.data_ptr()) % 16 == 0
                     and (bias is None or (bias.numel() == N and bias.is_contiguous() and bias.device == x.device))
                     and ops.direct_available()):
-                return ops.linear_w8a16_direct(x, x.numel() // K, K, weight, scale, rot, N, bias)
+                done = ops.linear_w8a16_direct(x, x.numel() // K, K, weight, scale, rot, N, bias)
+                if done is not None:
+                    return done
             rows = x.reshape(-1, self.in_features).contiguous()
             xr = ops.rotate_rows(rows, self.group_size) if self.convrot else rows
             y = ops.gemm_w8a16(xr, self.weight, self.weight_scale, bias, out_dtype=torch.float16)

@@ -7,6 +7,7 @@ on a tensor that is not on a GPU they raise ``RuntimeError``.
 """
 import contextlib
 import ctypes
+import threading
 
 import torch
 
@@ -346,21 +347,26 @@ def linear_w4a16_direct(x, M, K, wq, w_scale, w_zero, group_size, N, bias, into=
     return None if status else y
 
 
-# Flags of linear_w8a16, one per (device, stream), in pinned host memory with the last ticket handed
-# out: the kernel stores the ticket there when it finds a NaN or Inf, and the host reads it after
-# waiting for the stream -- no device-to-host copy.
+# Flags of linear_w8a16, one per (device, stream, thread), in pinned host memory with the last ticket
+# handed out: the kernel stores the ticket there when it finds a NaN or Inf, and the host reads it after
+# waiting for the stream -- no device-to-host copy.  The store does not keep a larger ticket, so threads
+# that share a stream have a flag each.  Calls past _MAX_FLAGS flags take the separate ops.
 _host_flags = {}
+_MAX_FLAGS = 64
 
 
 def linear_w8a16_direct(x, M, K, wq, w_scale, rot_group, N, bias):
     """Int8Linear's forward: x [..., K] and wq [N, K] contiguous, x f16/bf16, w_scale [N] fp32.  Returns
-    ([..., N], whether every output is finite) after waiting for the stream (1024 x 5120 x 5120 107.6 -> 92.0
-    us a forward, against rotate, GEMM, flag and read-back as separate calls)."""
+    ([..., N], whether every output is finite) after waiting for the stream, or None without a flag
+    (1024 x 5120 x 5120 107.6 -> 92.0 us a forward, against rotate, GEMM, flag and read-back as separate
+    calls)."""
     lib, dt, device = _native.lib(), _DT[x.dtype], x.device
     stream = _raw_stream(device.index)
-    key = (device.index, stream)
+    key = (device.index, stream, threading.get_ident())
     entry = _host_flags.get(key)
     if entry is None:
+        if len(_host_flags) >= _MAX_FLAGS:
+            return None
         flag = torch.zeros(1, dtype=torch.int64, pin_memory=True)
         entry = _host_flags[key] = [flag, 0, ctypes.c_uint64.from_address(flag.data_ptr())]
     ws, nb = _workspace(device, stream or None, lib.psq_gemm_wonly_workspace_bytes(_native.W_INT8, K, M, N, K, 0))

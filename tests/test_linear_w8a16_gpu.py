@@ -43,3 +43,25 @@ def test_one_call(gpu, M, N, K, dt, rot):
     if dt == torch.float16:
         assert not both(s * 1e6, b)          # ... and a sum past it rounds to infinity
     assert both(s, b)                        # a later finite call is finite again
+
+
+def test_flags_of_threads_and_their_bound(gpu, monkeypatch):
+    """Threads on one stream have a flag each; past the bound the separate ops answer."""
+    import threading
+    from powershard_amd import ops
+    x = torch.randn(4, 256, device=gpu).half()
+    wq = torch.randint(-127, 128, (64, 256), dtype=torch.int8, device=gpu)
+    s = torch.full((64,), 1e-3, device=gpu)
+    bad = torch.full((64,), float("inf"), device=gpu).half()
+    seen = {}
+
+    def work(i):
+        seen[i] = [ops.linear_w8a16_direct(x, 4, 256, wq, s, 256, 64, bad if (i + j) % 2 else None)[1] for j in range(50)]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert all(seen[i] == [(i + j) % 2 == 0 for j in range(50)] for i in range(4))
+    monkeypatch.setattr(ops, "_host_flags", {})
+    monkeypatch.setattr(ops, "_MAX_FLAGS", 0)
+    assert ops.linear_w8a16_direct(x, 4, 256, wq, s, 256, 64, None) is None
