@@ -30,7 +30,6 @@ constexpr int kMaxThreads = 1024;
 constexpr int kMaxChunks = 2;                                      // 16-element chunks per thread
 constexpr int kMaxK = kElemsPerThread * kMaxThreads * kMaxChunks;  // 32768
 
-
 // A workgroup quantizes R consecutive rows side by side (all their loads issued up front, one
 // shared barrier for the absmax reductions).  Thread t owns P chunks of 16 consecutive elements
 // of each row: chunk c = elements [(c T + lane_chunk(t)) 16, +16), T = blockDim.x (a multiple of
