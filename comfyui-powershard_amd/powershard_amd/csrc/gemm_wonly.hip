@@ -11,6 +11,7 @@
 // Two kernels: a weight-streaming one for M <= 64 (decode / short prompts: HBM-bound) and a
 // 256 x 256-tile one for larger M (MFMA-bound), both described where they are defined.
 #include "psq_common.hpp"
+#include "wonly_plan.hpp"
 
 #include <mutex>
 
@@ -19,8 +20,6 @@ namespace {
 
 constexpr int NTHREADS = 256;
 constexpr int KSTAGE = 64;                     // K granularity of every path
-
-enum { W_UINT4 = 0, W_INT8 = 1 };
 
 struct WArgs {
     const uint8_t *wq;          // uint4 [N, K/2] or int8 [N, K]
@@ -300,7 +299,7 @@ gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int
 // dequantization.  Lane-half h of every fragment carries k = 32 h + 8 t .. + 7 of the stage in
 // k-step t, for both operands, so a lane's weights of a stage are 16 contiguous bytes of nibbles.
 namespace wt {
-constexpr int BN = 256, BK = 64;
+constexpr int BN = kPlanBN, BK = kPlanBK;
 constexpr int TN = 1;                              // 32 x 32 tiles per wave: BM rows x 32 columns
 constexpr int WCOLS = 32 * TN;                     // output columns per wave
 constexpr int NWAVE = BN / WCOLS;                  // waves per workgroup (8: two per SIMD)
@@ -1842,90 +1841,6 @@ int launch_tiled_bm(const uint16_t *x, int64_t ldx, int64_t M, int64_t N, int64_
     return check_launch(name);
 }
 
-// Launch plan of the tiled kernel, in units of one 128-row tile's K stage on a lightly loaded GPU.
-//  * Data-parallel (one tile per workgroup): ceil(tiles / CUs) rounds of nk stages.  Tiles are 128,
-//    160, 192, 224 or 256 rows; a stage of theirs costs kRows[] of a 128-row one's (the
-//    dequantization serves all the rows: us a stage on 100 CUs, uint4, 0.86, 0.97, 1.02, 1.15, 1.25).
-//    The width in rows is the cheapest over the rounds it takes, so that a ragged M does not compute
-//    a mostly empty row tile: 300 x 25600 x 5120 125.1 us with two 256-row tiles, 93.0 with two of 160;
-//    384 x 25600 x 5120 127.5 -> 104.8 (192); 2048 x 25600 x 5120 529 -> 503 (224); f16 on int8 weights
-//    2048 x 5120 x 5120 109.2 -> 100.3 (192).
-//  * Stream-K, 128-row tiles only (the 256-row kernel has no registers to spare for it), over G
-//    workgroups: ceil(tiles nk / G) stages each.  With G a multiple s of the tiles, each workgroup
-//    takes one K range of one tile (one partial, written or added up); otherwise up to two
-//    segments (a second ring prologue, two partials).  Each partial costs about kSkPartCost.
-//  * The kernel is power-limited: with more than about 78% of the CUs busy the clock drops, a
-//    stage taking about 1 + 0.6 (busy fraction - 0.78) times as long (M=128 x N=25600: 1.13 us a
-//    stage on 200 CUs, 1.2-1.37 on 256).  f16 on int8 weights has so little dequantization that
-//    a stage on 160 CUs takes 0.75 us against 1.13 of stream-K on 256 (kSkStageF16I8): 1024 x 5120 x
-//    5120 64.6 us with stream-K, 59.7 with 160 whole tiles.
-// Stream-K is taken when it beats data-parallel by more than kSkMargin, and needs a workspace:
-// the tiles' arrival counters (kSkCntBytes, room for kSkMaxTiles) and two fp32 partial tiles per
-// workgroup.
-constexpr int kSkMinUnits = 8;                              // K stages per workgroup at least
-constexpr double kSkPartCost = 3.0, kSkRestartCost = 2.0, kSkMargin = 0.9;
-constexpr struct {
-    int bm;
-    double cost;
-} kRows[] = {{128, 1.0}, {160, 1.10}, {192, 1.17}, {224, 1.32}, {256, 1.44}};
-constexpr double kSkStageF16I8 = 1.4;
-constexpr int64_t kSkMaxTiles = 16384;
-constexpr int64_t kSkCntBytes = kSkMaxTiles * 4;
-constexpr int64_t kSkSlotBytes = 128LL * wt::BN * 4;        // one 128-row fp32 partial tile
-constexpr int kSkMaxGroups = 256;
-constexpr int64_t kMaxWsBytes = kSkCntBytes + 2 * kSkMaxGroups * kSkSlotBytes;   // 64 MB + 64 KB
-
-inline double clock_factor(int64_t busy, int cus)
-{
-    const double f = (double)busy / cus - 0.78;
-    return f > 0 ? 1.0 + 0.6 * f : 1.0;
-}
-
-struct TiledPlan {
-    int bm = 128;
-    int64_t tiles = 0;
-    int sk = 0;                 // stream-K workgroups (0: data-parallel)
-    int64_t ws_bytes = 0;
-};
-
-TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, int cus, bool allow_sk, double sk_stage = 1.0)
-{
-    TiledPlan p;
-    const int64_t nbn = (N + wt::BN - 1) / wt::BN, nk = K / wt::BK;
-    double t_dp = 0.0;
-    for (const auto &r : kRows) {
-        const int64_t tiles = ((M + r.bm - 1) / r.bm) * nbn;
-        const double t = (double)((tiles + cus - 1) / cus * nk) * r.cost * clock_factor(std::min<int64_t>(tiles, cus), cus);
-        if (p.tiles && t >= t_dp) continue;
-        t_dp = t;
-        p.bm = r.bm;
-        p.tiles = tiles;
-    }
-    if (!allow_sk) return p;
-    const int64_t t128 = ((M + 127) / 128) * nbn, units = t128 * nk;
-    if (t128 > kSkMaxTiles) return p;
-    double best = kSkMargin * t_dp;
-    int64_t best_g = 0;
-    auto consider = [&](int64_t g, bool aligned) {
-        if (g < 1 || g > cus || g > kSkMaxGroups || units / g < kSkMinUnits) return;
-        const double t = (double)((units + g - 1) / g) * clock_factor(g, cus) * sk_stage +
-                         (aligned ? kSkPartCost : 2 * kSkPartCost + kSkRestartCost);
-        if (t < best) {
-            best = t;
-            best_g = g;
-        }
-    };
-    for (int64_t sp = 2; t128 * sp <= cus; sp++) consider(t128 * sp, true);   // one K range of one tile each
-    consider(cus, false);
-    if (best_g) {
-        p.bm = 128;
-        p.tiles = t128;
-        p.sk = (int)best_g;
-        p.ws_bytes = kSkCntBytes + 2 * best_g * kSkSlotBytes;
-    }
-    return p;
-}
-
 // The weight-streaming kernel takes the uint4 shapes with M <= SKINNY_MAX_M and groups of a
 // multiple of 128; the skinny kernel takes M <= SKINNY_MAX_M when K is a whole number of
 // 128-element blocks (and, for uint4, the groups hold whole 32-element lane runs); the tiled
@@ -1943,7 +1858,7 @@ Path choose_path(int wk, int64_t ldx, int64_t M, int64_t N, int64_t K, int gs, b
         return Path::Decode;
     if (wk == W_UINT4 && M <= SKINNY_MAX_M && gs % 128 == 0 && K % ws::STEP == 0 && ldx <= (1LL << 22)) {
         if (ws && cus > 0 && 2 * ((N + ws::ROWS - 1) / ws::ROWS) <= cus && K >= 8192 && K <= (1LL << 22) &&
-            plan_tiled(M, N, K, cus, true).sk > 0)
+            plan_tiled(wk, PSQ_BF16, M, N, K, cus, true).sk > 0)
             return Path::Tiled;
         return Path::Stream;
     }
@@ -1951,7 +1866,7 @@ Path choose_path(int wk, int64_t ldx, int64_t M, int64_t N, int64_t K, int gs, b
     return Path::Tiled;
 }
 
-// Workspace bytes of a call (0: no split); the split needs a device, else 0.
+// Workspace bytes that cover a call of this shape (0: no split); the split needs a device, else 0.
 int64_t workspace_bytes(int wk, int64_t ldx, int64_t M, int64_t N, int64_t K, int gs)
 {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -1960,10 +1875,11 @@ int64_t workspace_bytes(int wk, int64_t ldx, int64_t M, int64_t N, int64_t K, in
     const int cus = cu_count(dev);
     const Path path = choose_path(wk, ldx, M, N, K, gs, true, cus);
     if (path != Path::Tiled) return 0;
-    return plan_tiled(M, N, K, cus, true).ws_bytes;
+    return plan_workspace(wk, M, N, K, cus);
 }
 
-// workspace: NULL = data-parallel tiles only; else at least workspace_bytes(), its counter words
+// workspace: NULL = data-parallel tiles only; else at least what the call's plan needs (at most
+// workspace_bytes()), its counter words
 // (the first kSkCntBytes) zero when first passed: every launch leaves them zero, and writes every
 // partial it reads.
 template <int WK>
@@ -1994,8 +1910,7 @@ int launch(const void *x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_
     }
     if (ldx > (1LL << 22)) return set_error(PSQ_E_SHAPE, "%s: ldx above 2^22", name);   // 32-bit row offsets
     if (K > (1LL << 22)) return set_error(PSQ_E_SHAPE, "%s: K above 2^22", name);       // (of the weights too)
-    const TiledPlan plan = plan_tiled(M, N, K, cu_count(dev), workspace != nullptr,
-                                      WK == W_INT8 && x_dtype == PSQ_F16 ? kSkStageF16I8 : 1.0);
+    const TiledPlan plan = plan_tiled(WK, x_dtype, M, N, K, cu_count(dev), workspace != nullptr);
     wa.sk = 0;
     if (plan.sk) {
         if (ws_bytes < plan.ws_bytes)

@@ -210,8 +210,8 @@ PSQ_API int psq_gemm_w8a16(const void *x, int x_dtype, int64_t ldx, const int8_t
                    int y_dtype, int64_t ldy, int64_t M, int64_t N, int64_t K, void *stream);
 
 /* Split-K workspace of the weight-only GEMMs.  When M, N and K leave CUs idle under the tiled
- * kernel (M > 64; e.g. M = 128 at N = 25600: 100 output tiles of 128 x 256 for 256 CUs, or M = 1024
- * at N = K = 5120: 160 tiles), the *_ws entry points split K across workgroups (stream-K): each
+ * kernel (M > 64; e.g. M = 128 at N = 25600, K = 5120: 100 output tiles of 128 x 256 for 256 CUs, or
+ * bf16 M = 1024 at N = K = 5120: 160 tiles), the *_ws entry points split K across workgroups (stream-K): each
  * tile's K range in a few equal parts, or the (tile, K stage) units of all tiles in equal runs
  * that cross tile boundaries.  A workgroup holding part of a tile writes its fp32 partial tile to
  * the workspace and counts itself in the tile's counter there; the last one to finish adds the
@@ -229,7 +229,8 @@ PSQ_API int psq_gemm_w8a16(const void *x, int x_dtype, int64_t ldx, const int8_t
  *                    calls that share it overlap (use one workspace per stream). */
 enum psq_weight_kind { PSQ_W_UINT4 = 0, PSQ_W_INT8 = 1 };
 
-/* Bytes of workspace a *_ws call of this shape uses on the current device (0: no split). */
+/* Bytes of workspace that cover a *_ws call of this shape on the current device with activations of
+ * either type (0: no split).  A call may use less: f16 activations on int8 weights split fewer shapes. */
 PSQ_API int64_t psq_gemm_wonly_workspace_bytes(int weight_kind, int64_t ldx, int64_t M, int64_t N, int64_t K,
                                                int group_size);
 PSQ_API int psq_gemm_w4a16_ws(const void *x, int x_dtype, int64_t ldx, const uint8_t *wq,
