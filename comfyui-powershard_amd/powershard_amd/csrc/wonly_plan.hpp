@@ -27,21 +27,22 @@ constexpr int kPlanBN = 256, kPlanBK = 64;                  // columns of a tile
 //    segments (a second ring prologue, two partials).  Each partial costs about kSkPartCost.
 //  * The kernel is power-limited: with more than about 78% of the CUs busy the clock drops, a
 //    stage taking about 1 + 0.6 (busy fraction - 0.78) times as long (M=128 x N=25600: 1.13 us a
-//    stage on 200 CUs, 1.2-1.37 on 256).  f16 on int8 weights has so little dequantization that
-//    a stage on 160 CUs takes 0.75 us against 1.13 of stream-K on 256 (kSkStageF16I8): 1024 x 5120 x
-//    5120 64.6 us with stream-K, 59.7 with 160 whole tiles.  That factor weighs the split against whole
-//    tiles only, not one split against another: G taken by it too was larger and slower (f16, 576 x
-//    5120 x 5120 256 workgroups 44.0 us, 200 43.3; 128 x 13824 x 13824 256 71.2, 216 64.4).
+//    stage on 200 CUs, 1.2-1.37 on 256).
 // Stream-K is taken when it beats data-parallel by more than kSkMargin, and needs a workspace:
 // the tiles' arrival counters (kSkCntBytes, room for kSkMaxTiles) and two fp32 partial tiles per
-// workgroup.
+// workgroup.  f16 on int8 weights has so little dequantization that its stages are short beside the
+// partials: there the same split is taken when it saves kSkF16I8 stages (one K range of one tile per
+// workgroup) or kSkF16I8Runs (runs across tiles).  Measured (us, whole tiles against the split, over 150
+// shapes the two meet at these savings): 8 stages saved, 679 x 4096 x 1024 15.4 / 20.6; 24, 202 x 1137 x
+// 2048 31.7 / 28.0; runs, 19, 1024 x 5120 x 5120 55.8 / 58.1; 26, 383 x 14336 x 6656 85.1 / 78.2; 81, 827 x
+// 5120 x 13824 141.7 / 122.6.
 constexpr int kSkMinUnits = 8;                              // K stages per workgroup at least
 constexpr double kSkPartCost = 3.0, kSkRestartCost = 2.0, kSkMargin = 0.9;
 constexpr struct {
     int bm;
     double cost;
 } kRows[] = {{128, 1.0}, {160, 1.10}, {192, 1.17}, {224, 1.32}, {256, 1.44}};
-constexpr double kSkStageF16I8 = 1.4;
+constexpr double kSkF16I8 = 17.0, kSkF16I8Runs = 28.0;
 constexpr int64_t kSkMaxTiles = 16384;
 constexpr int64_t kSkCntBytes = kSkMaxTiles * 4;
 constexpr int64_t kSkSlotBytes = 128LL * kPlanBN * 4;       // one 128-row fp32 partial tile
@@ -64,7 +65,6 @@ struct TiledPlan {
 // The plan of a call: weight kind wk, activations of x_dtype (PSQ_BF16 or PSQ_F16).
 inline TiledPlan plan_tiled(int wk, int x_dtype, int64_t M, int64_t N, int64_t K, int cus, bool allow_sk)
 {
-    const double sk_stage = wk == W_INT8 && x_dtype == PSQ_F16 ? kSkStageF16I8 : 1.0;
     TiledPlan p;
     const int64_t nbn = (N + kPlanBN - 1) / kPlanBN, nk = K / kPlanBK;
     double t_dp = 0.0;
@@ -79,21 +79,24 @@ inline TiledPlan plan_tiled(int wk, int x_dtype, int64_t M, int64_t N, int64_t K
     if (!allow_sk) return p;
     const int64_t t128 = ((M + 127) / 128) * nbn, units = t128 * nk;
     if (t128 > kSkMaxTiles) return p;
-    double best = 1e300, extra = 0.0;
+    double best = 1e300, saved = 0.0;
     int64_t best_g = 0;
+    bool runs = false;
     auto consider = [&](int64_t g, bool aligned) {
         if (g < 1 || g > cus || g > kSkMaxGroups || units / g < kSkMinUnits) return;
         const double stages = (double)((units + g - 1) / g) * clock_factor(g, cus);
         const double t = stages + (aligned ? kSkPartCost : 2 * kSkPartCost + kSkRestartCost);
         if (t < best) {
             best = t;
-            extra = (sk_stage - 1.0) * stages;
+            saved = t_dp - stages;
+            runs = !aligned;
             best_g = g;
         }
     };
     for (int64_t sp = 2; t128 * sp <= cus; sp++) consider(t128 * sp, true);   // one K range of one tile each
     consider(cus, false);
-    if (best_g && best + extra < kSkMargin * t_dp) {
+    const bool pays = wk == W_INT8 && x_dtype == PSQ_F16 ? saved > (runs ? kSkF16I8Runs : kSkF16I8) : true;
+    if (best_g && best < kSkMargin * t_dp && pays) {
         p.bm = 128;
         p.tiles = t128;
         p.sk = (int)best_g;

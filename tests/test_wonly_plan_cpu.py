@@ -63,8 +63,10 @@ def test_query_covers_every_launch(plan, cus):
 
 
 @pytest.mark.parametrize("M,N,K,split", [(576, 5120, 5120, True), (700, 4096, 4096, True), (128, 13824, 13824, True),
-                                         (1024, 5120, 5120, False), (2500, 2048, 5376, False)])
+                                         (827, 5120, 13824, True), (202, 1137, 2048, True), (1081, 5120, 25600, True),
+                                         (1024, 5120, 5120, False), (2500, 2048, 5376, False), (69, 4608, 1024, False)])
 def test_f16_splits_as_bf16_or_not_at_all(plan, M, N, K, split):
-    """f16 on int8 weights: bf16's split, or whole tiles (and then the query still covers bf16)."""
+    """f16 on int8 weights: bf16's split where it measured faster, else whole tiles (and then the query
+    still covers bf16)."""
     bf16, f16 = (plan.need(1, dt, M, N, K, 256) for dt in (0, 1))
     assert f16 == (bf16 if split else 0) and 0 < bf16 == plan.told(1, M, N, K, 256) <= plan.most()
