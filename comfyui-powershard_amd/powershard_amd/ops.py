@@ -315,23 +315,52 @@ def gemm_w8a16(x, wq, w_scale, bias=None, out_dtype=None):
 # The launches of a QuantLinear forward with nothing to convert: addresses and sizes straight to the
 # library, at most one scratch allocation, no tensor per stored component.  For the small calls, which
 # the host bounds: an int8 or fp8 forward 39 -> 17.8 us of host time (one or two rows, quantized inside
-# the GEMM: 13.8 us), int4 28 -> 13.5 us.  The
-# arguments are as the general ops check them (QuantLinear._direct); None when the library refuses,
-# and the caller's general path then reports why.
+# the GEMM: 13.8 us), int4 28 -> 13.5 us.  The arguments are as the general ops check them
+# (QuantLinear._direct); None when the library refuses, and the caller's general path then reports why.
+def quantized_in_gemm(M, K, act):
+    """Whether linear_q8_direct quantizes the rows inside its GEMM (no codes, no scratch: psq_linear_q8)."""
+    return M <= 2 and K <= 8192 and act != ACTIVATIONS["silu_gate"]
+
+
 def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, act, into=None):
     """x [..., K] contiguous bf16/f16; w, w_scale: device addresses.  [..., N] (gate: N / 2) of x's
     dtype; into: [M, N] rows of x's dtype or fp32 (the same values) that take the result."""
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
     y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device) if into is None else into
-    # (one or two rows are quantized inside the GEMM: no scratch, see psq_linear_q8)
-    scratch = None if M <= 2 and K <= 8192 and act != ACTIVATIONS["silu_gate"] else \
+    scratch = None if quantized_in_gemm(M, K, act) else \
         torch.empty(((M * K + 15) & -16) + 4 * M, dtype=torch.uint8, device=x.device)
     status = lib.psq_linear_q8(weights, x.data_ptr(), dt, K, rot_group, w, K, w_scale, per_row,
                                None if bias is None else bias.data_ptr(), dt, act, y.data_ptr(),
                                int(y.dtype is torch.float32), cols, M, N, K,
                                None if scratch is None else scratch.data_ptr(),
                                _raw_stream(x.device.index))
+    return None if status else y
+
+
+def quantize_direct(x, M, K, fp8, rot_group):
+    """quantize_rows of x [..., K] contiguous bf16/f16: (codes [M, K], scales [M])."""
+    lib = _native.lib()
+    q = torch.empty(M, K, dtype=torch.float8_e4m3fn if fp8 else torch.int8, device=x.device)
+    scale = torch.empty(M, dtype=torch.float32, device=x.device)
+    status = (lib.psq_quantize_rows_fp8 if fp8 else lib.psq_quantize_rows_i8)(
+        x.data_ptr(), _DT[x.dtype], M, K, K, rot_group, None, q.data_ptr(), K, scale.data_ptr(), _raw_stream(x.device.index))
+    return None if status else (q, scale)
+
+
+def linear_codes_direct(x, q, scale, M, K, weights, w, w_scale, per_row, N, bias, act):
+    """linear_q8_direct of rows that are quantized already (q, scale: quantize_direct of x)."""
+    lib, dt = _native.lib(), _DT[x.dtype]
+    cols = _out_cols(N, act, "linear_q8")
+    y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device)
+    b = None if bias is None else bias.data_ptr()
+    out = (y.data_ptr(), dt, cols, M, N, K, _raw_stream(x.device.index))
+    if weights == _native.Q8_I8:
+        status = lib.psq_gemm_i8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, b, dt, act, *out)
+    elif weights == _native.Q8_E4M3:
+        status = lib.psq_gemm_fp8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, b, dt, act, *out)
+    else:
+        status = lib.psq_gemm_fp8_e5m2w(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, b, dt, *out)
     return None if status else y
 
 

@@ -336,15 +336,14 @@ class QuantLinear(nn.Module):
 
     def _direct(self, x, activation, into=None):
         """The native forward in one library call, or None where anything has to be converted,
-        copied, shared, tracked, timed or refused: the general path below takes those (and reports
-        what the library refuses).  Same kernels, same values."""
+        copied, tracked, timed or refused: the general path below takes those (and reports what the
+        library refuses).  Rows that reuse_quantized_inputs shares are quantized in a call of their
+        own.  Same kernels, same values."""
         own = self.__dict__
         dtype = self._ps_compute_dtype
         if (not self._ps_native or self._ps_full_precision or type(x) is not torch.Tensor or not x.is_cuda
                 or x.dtype is not dtype or (dtype is not torch.bfloat16 and dtype is not torch.float16)
-                or self._modules or own.get("_ps_safe") or own.get("_ps_tracker") is not None
-                or (getattr(_shared, "cache", None) is not None and x.numel() > _SHARE_ELEMENTS
-                    and x.numel() * self.out_features > _SHARE_PRODUCTS)):
+                or self._modules or own.get("_ps_safe") or own.get("_ps_tracker") is not None):
             return None
         from . import ops
         plan, store, bias = self._ps_qplan, self.qbytes, self.bias
@@ -388,8 +387,14 @@ class QuantLinear(nn.Module):
         if into is not None and ((into.dtype is not dtype and (into.dtype is not torch.float32 or weights == 2))
                                  or not _takes(into, device, M, N)):
             into = None
-        return ops.linear_q8_direct(x, M, K, weights, base + q_at, base + s_at, int(count > 1), rot, N, bias,
-                                    ops.ACTIVATIONS[activation], into)
+        act = ops.ACTIVATIONS[activation]
+        cache = getattr(_shared, "cache", None)
+        # an MLP's hidden rows (into) go to one module only, and one or two rows cost the GEMM nothing
+        if cache is not None and into is None and not ops.quantized_in_gemm(M, K, act):
+            codes = _shared_codes(cache, x, M, K, weights != 0, rot)
+            return None if codes is None else ops.linear_codes_direct(
+                x, *codes, M, K, weights, base + q_at, base + s_at, int(count > 1), N, bias, act)
+        return ops.linear_q8_direct(x, M, K, weights, base + q_at, base + s_at, int(count > 1), rot, N, bias, act, into)
 
     def _forward(self, x, activation, into=None):
         if self._ps_native:
@@ -424,10 +429,6 @@ def _takes(into, device, M, N):
 
 # ------------------------------------------------------------------ shared activation quantization
 _shared = threading.local()
-# Calls up to these sizes are quantized by each module's one-call forward, also where they could be
-# shared: quantizing 4M elements again takes about 5 us, and a GEMM of 2^35 products about 30 us, the host
-# time of the general path that shares (q, k and v of 3022 x 1024, 64 columns each: 109.9 -> 47.5 us).
-_SHARE_ELEMENTS, _SHARE_PRODUCTS = 1 << 22, 1 << 35
 
 
 @contextlib.contextmanager
@@ -435,6 +436,7 @@ def reuse_quantized_inputs():
     """Within the block, native W8A8 / FP8 modules that receive the same activation tensor quantize
     it once: the q, k and v projections of one attention input (three QuantLinear calls on the same
     x in the reference's Wan block, each quantizing x itself) share one rotate + quantize pass.
+    (One or two rows are quantized inside each module's GEMM instead, which takes no longer.)
 
     A quantized input is reused only for the same storage, offset, shape, strides, dtype and
     in-place version of the rows tensor, the same rotation group / format / static scale, and the
@@ -452,24 +454,42 @@ def reuse_quantized_inputs():
         _shared.cache = prev
 
 
+def _input_key(rows, shape, strides, fp8, group, input_scale):
+    """What a quantized input is known by: rows' memory laid out as `shape`, `strides`."""
+    from . import ops
+    try:
+        version = rows._version
+    except RuntimeError:   # inference tensors (torch.inference_mode) carry no version counter
+        version = None
+    return (rows.data_ptr(), tuple(shape), tuple(strides), rows.dtype, version, bool(fp8), int(group or 0),
+            None if input_scale is None else (input_scale.data_ptr(), input_scale._version), ops._stream(rows).value)
+
+
+def _shared_codes(cache, x, M, K, fp8, group):
+    """(codes, scales) of the rows of x [..., K] contiguous for the one-call forward: those that a
+    module of this block made, else new ones for the next module.  None when the library refuses."""
+    from . import ops
+    key = _input_key(x, (M, K), (K, 1), fp8, group, None)
+    hit = cache.get(key)
+    if hit is None:
+        codes = ops.quantize_direct(x, M, K, fp8, group)
+        if codes is None:
+            return None
+        hit = cache[key] = (x, *codes, None)   # the references keep the keyed memory alive
+    return hit[1], hit[2]
+
+
 def _quantize_input(rows, fp8, group, input_scale):
     from . import ops
     cache = getattr(_shared, "cache", None)
     if cache is None:
         return ops.quantize_rows(rows, fp8=fp8, rot_group=group, static_scale=input_scale)
-    try:
-        version = rows._version
-    except RuntimeError:   # inference tensors (torch.inference_mode) carry no version counter
-        version = None
-    key = (rows.data_ptr(), tuple(rows.shape), tuple(rows.stride()), rows.dtype, version, bool(fp8),
-           int(group or 0), None if input_scale is None else (input_scale.data_ptr(), input_scale._version),
-           torch.cuda.current_stream(rows.device).cuda_stream)
+    key = _input_key(rows, rows.shape, rows.stride(), fp8, group, input_scale)
     hit = cache.get(key)
-    if hit is not None:
-        return hit[1], hit[2]
-    qx, sx = ops.quantize_rows(rows, fp8=fp8, rot_group=group, static_scale=input_scale)
-    cache[key] = (rows, qx, sx, input_scale)   # the references keep the keyed memory alive
-    return qx, sx
+    if hit is None:
+        qx, sx = ops.quantize_rows(rows, fp8=fp8, rot_group=group, static_scale=input_scale)
+        hit = cache[key] = (rows, qx, sx, input_scale)   # the references keep the keyed memory alive
+    return hit[1], hit[2]
 
 
 def apply_activation(out, activation):
