@@ -70,14 +70,14 @@ class Int8Linear(nn.Module):
             # The kernel path rounds x H to fp16, and |x H| reaches sqrt(g) max|x| where coherent
             # activations line up with a row of H; the tile path never forms x H.  A non-finite
             # kernel output is therefore recomputed on the tiles before it is reported or raised.
-            # That decision reads the output's flag back (an 8-byte read, a synchronization) on
-            # every call, also with a finite tracker attached, whose own checks the reference
-            # defers to one read per forward (fp16_safe.py FiniteTracker.finish): the tracker must
-            # not see an overflow the tile path would not have produced.
+            # That decision waits for the stream on every call (the GEMM raises a flag in host memory;
+            # the separate ops read an 8-byte flag back), also with a finite tracker attached, whose
+            # own checks the reference defers to one read per forward (fp16_safe.py
+            # FiniteTracker.finish): the tracker must not see an overflow the tile path would not have
+            # produced.  An error that the wait reports is raised: it says nothing about the shape.
             if out is not None:
-                out, finite = out
-                if finite is None:
-                    finite = not ops.any_nonfinite(out)
+                out, pending = out
+                finite = not ops.any_nonfinite(out) if pending is None else ops.linear_w8a16_finite(pending)
                 if not finite:
                     out = None
         if out is None:
@@ -105,12 +105,12 @@ class Int8Linear(nn.Module):
         return getattr(self, "_ps_safe", False) or self.weight.device.type != "cuda" or not getattr(self, "_ps_native", True)
 
     def _native_forward(self, x, check):
-        """fp16 x [..., K] -> (fp16 [..., N], whether it is finite, None where that is still to be
-        checked) on the gfx950 kernels, or None (and the tile path from then on) when the kernels do
-        not take the shape.  A missing library raises (as on the tile
-        path, whose GPU dequantization is a kernel too).  The dequantized weight's fp16 range check
-        of the tile path (dequantize_rows) is kept as a bound, once: every element of (q s) H^T is
-        at most sqrt(g) max|q s| in magnitude."""
+        """fp16 x [..., K] -> (fp16 [..., N], the output check that its launches raise, None where it
+        is a call of its own) on the gfx950 kernels, or None (and the tile path from then on) when the
+        kernels do not take the shape.  A missing library raises (as on the tile path, whose GPU
+        dequantization is a kernel too).  The dequantized weight's fp16 range check of the tile path
+        (dequantize_rows) is kept as a bound, once: every element of (q s) H^T is at most
+        sqrt(g) max|q s| in magnitude."""
         from . import ops
         if check and not getattr(self, "_ps_range_ok", False):
             bound = (self.weight.abs().amax(dim=1, keepdim=True).float() * self.weight_scale.float().abs()).max()
@@ -130,7 +130,7 @@ class Int8Linear(nn.Module):
                     and scale.device == x.device and (x.data_ptr() | weight.data_ptr()) % 16 == 0
                     and (bias is None or (bias.numel() == N and bias.is_contiguous() and bias.device == x.device))
                     and ops.direct_available()):
-                done = ops.linear_w8a16_direct(x, x.numel() // K, K, weight, scale, rot, N, bias)
+                done = ops.linear_w8a16_launch(x, x.numel() // K, K, weight, scale, rot, N, bias)
                 if done is not None:
                     return done
             rows = x.reshape(-1, self.in_features).contiguous()

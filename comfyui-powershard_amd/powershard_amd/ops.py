@@ -384,11 +384,9 @@ _host_flags = {}
 _MAX_FLAGS = 64
 
 
-def linear_w8a16_direct(x, M, K, wq, w_scale, rot_group, N, bias):
-    """Int8Linear's forward: x [..., K] and wq [N, K] contiguous, x f16/bf16, w_scale [N] fp32.  Returns
-    ([..., N], whether every output is finite) after waiting for the stream, or None without a flag
-    (1024 x 5120 x 5120 107.6 -> 92.0 us a forward, against rotate, GEMM, flag and read-back as separate
-    calls)."""
+def linear_w8a16_launch(x, M, K, wq, w_scale, rot_group, N, bias):
+    """Int8Linear's launches: x [..., K] and wq [N, K] contiguous, x f16/bf16, w_scale [N] fp32.
+    ([..., N], the check that linear_w8a16_finite answers), or None without a flag."""
     lib, dt, device = _native.lib(), _DT[x.dtype], x.device
     stream = _raw_stream(device.index)
     key = (device.index, stream, threading.get_ident())
@@ -406,8 +404,22 @@ def linear_w8a16_direct(x, M, K, wq, w_scale, rot_group, N, bias):
         x.data_ptr(), dt, K, rot_group, wq.data_ptr(), w_scale.data_ptr(), None if bias is None else bias.data_ptr(), dt,
         y.data_ptr(), N, M, N, K, None if rotated is None else rotated.data_ptr(),
         None if ws is None else ws.data_ptr(), nb, entry[0].data_ptr(), ticket, stream), "linear_w8a16")
+    return y, (device, entry, ticket)
+
+
+def linear_w8a16_finite(check):
+    """Whether every output of the launch is finite, after waiting for the stream.  An error that the
+    wait reports (of this work or of earlier work on the stream) is the caller's."""
+    device, entry, ticket = check
     torch.cuda.current_stream(device).synchronize()
-    return y, entry[2].value < ticket
+    return entry[2].value < ticket
+
+
+def linear_w8a16_direct(x, M, K, wq, w_scale, rot_group, N, bias):
+    """Launch and check: ([..., N], whether every output is finite), or None (1024 x 5120 x 5120 107.6 ->
+    92.0 us a forward, against rotate, GEMM, flag and read-back as separate calls)."""
+    done = linear_w8a16_launch(x, M, K, wq, w_scale, rot_group, N, bias)
+    return None if done is None else (done[0], linear_w8a16_finite(done[1]))
 
 
 def direct_available():

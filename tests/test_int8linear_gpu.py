@@ -118,3 +118,21 @@ def test_any_nonfinite_matches_torch(gpu, dtype, n, offset):
             assert ops.any_nonfinite(t), (pos, bad)
             t[pos] = keep
             assert not ops.any_nonfinite(t), (pos, bad, "after")
+
+
+def test_int8linear_error_of_the_wait_is_raised(gpu, monkeypatch):
+    """An error that the wait for the stream reports (a device error of earlier work) reaches the caller,
+    and is not taken for a shape that the kernels refuse."""
+    layer = make(256, 64, True, 256, gpu, seed=11)
+    x = (torch.randn(4, 256, generator=seeded(12)) * 0.5).half().to(gpu)
+    ref = layer(x)
+
+    def fail(self):
+        raise RuntimeError("reported by the wait")
+
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda.Stream, "synchronize", fail)
+        with pytest.raises(RuntimeError, match="reported by the wait"):
+            layer(x)
+    assert getattr(layer, "_ps_native", True)
+    assert torch.equal(layer(x).view(torch.int16), ref.view(torch.int16))
