@@ -18,6 +18,7 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
+from .quant_linear import PLAIN
 from .quant_tensor import regular_hadamard as _hadamard
 
 
@@ -124,7 +125,9 @@ class Int8Linear(nn.Module):
         weight, scale, rot = self.weight, self.weight_scale, self.group_size if self.convrot else 0
         N, K = weight.shape
         try:
-            if (type(x) is torch.Tensor and x.numel() and x.shape[-1] == K == self.in_features and x.is_contiguous()
+            if (type(x) is torch.Tensor and type(weight) in PLAIN and type(scale) in PLAIN
+                    and (bias is None or type(bias) in PLAIN)
+                    and x.numel() and x.shape[-1] == K == self.in_features and x.is_contiguous()
                     and weight.dtype is torch.int8 and weight.is_contiguous() and weight.device == x.device
                     and scale.dtype is torch.float32 and scale.is_contiguous() and scale.numel() == N
                     and scale.device == x.device and (x.data_ptr() | weight.data_ptr()) % 16 == 0

@@ -49,7 +49,7 @@ NATIVE = {"int8_tensorwise": "gemm_i8", "float8_e4m3fn": "gemm_fp8", "float8_e5m
 # stored code type -> the library's weight kind (enum psq_q8_weights)
 _Q8_WEIGHTS = {torch.int8: 0, torch.float8_e4m3fn: 1, torch.float8_e5m2: 2}
 # tensors whose memory is what their attributes say (no sharded or wrapping subclass)
-_PLAIN = (torch.Tensor, nn.Parameter)
+PLAIN = (torch.Tensor, nn.Parameter)
 # The exceptions of a native attempt that switch a module to dequantize (quant_linear.py:207-215).
 NATIVE_FAILURES = (NotImplementedError, RuntimeError, TypeError, ValueError)
 
@@ -355,8 +355,8 @@ class QuantLinear(nn.Module):
         if uint4:
             K *= 2
         numel, device = x.numel(), x.device
-        if (not numel or x.shape[-1] != K or not x.is_contiguous() or name != "scale" or type(store) not in _PLAIN
-                or (bias is not None and type(bias) not in _PLAIN) or store.device != device
+        if (not numel or x.shape[-1] != K or not x.is_contiguous() or name != "scale" or type(store) not in PLAIN
+                or (bias is not None and type(bias) not in PLAIN) or store.device != device
                 or store.dtype is not torch.uint8 or store.dim() != 1 or store.numel() < plan.total
                 or not store.is_contiguous() or not ops.direct_available()):
             return None

@@ -568,3 +568,32 @@ def test_rows2d_packs_what_the_kernels_cannot_address():
     packed = cases["packed"]
     assert _rows2d(packed).data_ptr() == packed.data_ptr()          # no copy when not needed
     assert _rows2d(torch.empty(0, 256)).shape == (0, 256)
+
+
+class _Sharded(torch.nn.Parameter):
+    """A parameter subclass: its attributes may describe more than its memory holds."""
+
+
+@pytest.mark.parametrize("name", [None, "weight", "weight_scale", "bias"])
+def test_int8linear_addresses_of_plain_tensors_only(monkeypatch, name):
+    """Int8Linear's one-call forward reads its tensors by address: a parameter subclass is left to the
+    separate ops (here, without a GPU, those raise and the module keeps its tiles)."""
+    from powershard_amd import ops
+    src = torch.nn.Linear(256, 32).half()
+    layer = Int8Linear(src, dict(convrot=True, group_size=256), rows=8).to_empty(device="cpu")
+    for p in layer.parameters():
+        p.data.zero_()
+    if name is not None:
+        setattr(layer, name, _Sharded(getattr(layer, name).data, requires_grad=False))
+    launched = []
+
+    def launch(x, M, K, *args):
+        launched.append((M, K))
+        return x.new_zeros(M, 32), "check"
+
+    monkeypatch.setattr(ops, "linear_w8a16_launch", launch)
+    out = layer._native_forward(torch.zeros(3, 256, dtype=torch.float16), check=False)
+    if name is None:
+        assert launched == [(3, 256)] and out[1] == "check"
+    else:
+        assert launched == [] and out is None and layer._ps_native is False
