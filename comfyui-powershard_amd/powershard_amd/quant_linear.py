@@ -360,8 +360,14 @@ class QuantLinear(nn.Module):
                 or store.dtype is not torch.uint8 or store.dim() != 1 or store.numel() < plan.total
                 or not store.is_contiguous() or not ops.direct_available()):
             return None
-        base, M = store.data_ptr(), numel // K
-        if (base | x.data_ptr()) % 16 or (bias is not None and (
+        try:
+            base, start = store.data_ptr(), x.data_ptr()
+            if bias is not None:
+                bias.data_ptr()
+        except RuntimeError:   # no memory of its own (vmap)
+            return None
+        M = numel // K
+        if (base | start) % 16 or (bias is not None and (
                 bias.dtype is not dtype or bias.device != device or bias.numel() != N or not bias.is_contiguous())):
             return None
         if uint4:
@@ -398,12 +404,7 @@ class QuantLinear(nn.Module):
 
     def _forward(self, x, activation, into=None):
         if self._ps_native:
-            try:
-                out = self._direct(x, activation, into)
-            except torch.cuda.OutOfMemoryError:
-                raise
-            except NATIVE_FAILURES:   # e.g. a tensor without storage (vmap): the general path's policy applies
-                out = None
+            out = self._direct(x, activation, into)
             if out is not None:
                 return out
         dtype = self._dtype_for(x)
