@@ -68,7 +68,7 @@ struct Finite {
     }
     __device__ __forceinline__ void report(const WArgs &wa) const
     {
-        // a plain store (the flag may be host memory): the flag has one caller, whose tickets grow
+        // a plain store (the flag may be host memory): the flag serves one call at a time, with growing tickets
         if (wa.flag && (bad & 0x80008000u)) __hip_atomic_store(wa.flag, wa.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 };

@@ -376,12 +376,34 @@ def linear_w4a16_direct(x, M, K, wq, w_scale, w_zero, group_size, N, bias, into=
     return None if status else y
 
 
-# Flags of linear_w8a16, one per (device, stream, thread), in pinned host memory with the last ticket
-# handed out: the kernel stores the ticket there when it finds a NaN or Inf, and the host reads it after
-# waiting for the stream -- no device-to-host copy.  The store does not keep a larger ticket, so threads
-# that share a stream have a flag each.  Calls past _MAX_FLAGS flags take the separate ops.
+# Flags of linear_w8a16 in pinned host memory, each with the last ticket handed out: the kernel stores
+# the ticket there when it finds a NaN or Inf, and the host reads it after waiting for the stream -- no
+# device-to-host copy.  The store does not keep a larger ticket, so a flag serves one call at a time: a
+# call takes one that no call holds and gives it back once its stream was waited for (a call that
+# failed in between keeps it: its kernel may still write there).  {device index: (all, free)}; a device
+# has as many as calls ran on it at once, at most _MAX_FLAGS, and a call without one takes the separate
+# ops.
 _host_flags = {}
 _MAX_FLAGS = 64
+_flags_lock = threading.Lock()
+
+
+def _take_flag(index):
+    with _flags_lock:
+        made, free = _host_flags.setdefault(index, ([], []))
+        if free:
+            return free.pop()
+        if len(made) >= _MAX_FLAGS:
+            return None
+        flag = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+        made.append([flag, 0, ctypes.c_uint64.from_address(flag.data_ptr())])
+        return made[-1]
+
+
+def _give_flag(index, entry):
+    with _flags_lock:
+        if index in _host_flags:
+            _host_flags[index][1].append(entry)
 
 
 def linear_w8a16_launch(x, M, K, wq, w_scale, rot_group, N, bias):
@@ -389,21 +411,21 @@ def linear_w8a16_launch(x, M, K, wq, w_scale, rot_group, N, bias):
     ([..., N], the check that linear_w8a16_finite answers), or None without a flag."""
     lib, dt, device = _native.lib(), _DT[x.dtype], x.device
     stream = _raw_stream(device.index)
-    key = (device.index, stream, threading.get_ident())
-    entry = _host_flags.get(key)
-    if entry is None:
-        if len(_host_flags) >= _MAX_FLAGS:
-            return None
-        flag = torch.zeros(1, dtype=torch.int64, pin_memory=True)
-        entry = _host_flags[key] = [flag, 0, ctypes.c_uint64.from_address(flag.data_ptr())]
     ws, nb = _workspace(device, stream or None, lib.psq_gemm_wonly_workspace_bytes(_native.W_INT8, K, M, N, K, 0))
     y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=device)
     rotated = torch.empty(M, K, dtype=x.dtype, device=device) if rot_group else None
+    entry = _take_flag(device.index)
+    if entry is None:
+        return None
     entry[1] = ticket = entry[1] + 1
-    _native.check(lib.psq_linear_w8a16(
-        x.data_ptr(), dt, K, rot_group, wq.data_ptr(), w_scale.data_ptr(), None if bias is None else bias.data_ptr(), dt,
-        y.data_ptr(), N, M, N, K, None if rotated is None else rotated.data_ptr(),
-        None if ws is None else ws.data_ptr(), nb, entry[0].data_ptr(), ticket, stream), "linear_w8a16")
+    try:
+        _native.check(lib.psq_linear_w8a16(
+            x.data_ptr(), dt, K, rot_group, wq.data_ptr(), w_scale.data_ptr(), None if bias is None else bias.data_ptr(), dt,
+            y.data_ptr(), N, M, N, K, None if rotated is None else rotated.data_ptr(),
+            None if ws is None else ws.data_ptr(), nb, entry[0].data_ptr(), ticket, stream), "linear_w8a16")
+    except Exception:   # refused: the GEMM was not launched
+        _give_flag(device.index, entry)
+        raise
     return y, (device, entry, ticket)
 
 
@@ -412,7 +434,9 @@ def linear_w8a16_finite(check):
     wait reports (of this work or of earlier work on the stream) is the caller's."""
     device, entry, ticket = check
     torch.cuda.current_stream(device).synchronize()
-    return entry[2].value < ticket
+    finite = entry[2].value < ticket
+    _give_flag(device.index, entry)
+    return finite
 
 
 def linear_w8a16_direct(x, M, K, wq, w_scale, rot_group, N, bias):

@@ -247,7 +247,8 @@ PSQ_API int psq_gemm_w8a16_ws(const void *x, int x_dtype, int64_t ldx, const int
  * `rotated` ([M, K] of x_dtype, 16-byte aligned; unused for rot_group 0), psq_gemm_w8a16_ws of the
  * rows, output of x_dtype, and the output check of psq_flag_nonfinite in the GEMM's epilogue: *flag
  * (device memory, or host memory that the device can write) becomes `ticket` when an output is NaN or
- * +-Inf (a plain store).  One flag per stream and calling thread, tickets from 1 and increasing. */
+ * +-Inf (a plain store).  A flag serves one call at a time: pass it again after waiting for its last
+ * call, with a larger ticket (from 1). */
 PSQ_API int psq_linear_w8a16(const void *x, int x_dtype, int64_t ldx, int rot_group, const int8_t *wq,
                      const float *w_scale, const void *bias, int bias_dtype, void *y, int64_t ldy,
                      int64_t M, int64_t N, int64_t K, void *rotated, void *workspace,

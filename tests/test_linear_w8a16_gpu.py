@@ -46,7 +46,7 @@ def test_one_call(gpu, M, N, K, dt, rot):
 
 
 def test_flags_of_threads_and_their_bound(gpu, monkeypatch):
-    """Threads on one stream have a flag each; past the bound the separate ops answer."""
+    """Calls that run at once have a flag each; past the bound the separate ops answer."""
     import threading
     from powershard_amd import ops
     x = torch.randn(4, 256, device=gpu).half()
@@ -65,3 +65,44 @@ def test_flags_of_threads_and_their_bound(gpu, monkeypatch):
     monkeypatch.setattr(ops, "_host_flags", {})
     monkeypatch.setattr(ops, "_MAX_FLAGS", 0)
     assert ops.linear_w8a16_direct(x, 4, 256, wq, s, 256, 64, None) is None
+
+
+def test_flags_are_given_back(gpu, monkeypatch):
+    """More threads than flags, all alive, one call each at a time: one flag serves them all.  A refused
+    call gives its flag back, one whose wait failed does not (its kernel may still write there)."""
+    import threading
+    from powershard_amd import ops
+    monkeypatch.setattr(ops, "_host_flags", {})
+    x = torch.randn(4, 256, device=gpu).half()
+    wq = torch.randint(-127, 128, (64, 256), dtype=torch.int8, device=gpu)
+    s = torch.full((64,), 1e-3, device=gpu)
+    one, done, seen = threading.Lock(), threading.Event(), []
+
+    def work():
+        with one:
+            seen.append(ops.linear_w8a16_direct(x, 4, 256, wq, s, 256, 64, None))
+        done.wait(60)
+
+    threads = [threading.Thread(target=work) for _ in range(ops._MAX_FLAGS + 6)]
+    [t.start() for t in threads]
+    while len(seen) < len(threads) and any(t.is_alive() for t in threads):
+        threads[0].join(0.01)
+    done.set()
+    [t.join() for t in threads]
+    assert len(seen) == len(threads) and all(r is not None and r[1] for r in seen)
+    made, free = ops._host_flags[gpu.index]
+    assert len(made) == len(free) == 1
+    with pytest.raises(RuntimeError):            # 96 elements are not whole 64-element stages
+        ops.linear_w8a16_direct(x[:, :96].contiguous(), 4, 96, wq[:, :96].contiguous(), s, 0, 64, None)
+    assert len(made) == len(free) == 1
+
+    def fail(self):
+        raise RuntimeError("reported by the wait")
+
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda.Stream, "synchronize", fail)
+        with pytest.raises(RuntimeError, match="by the wait"):
+            ops.linear_w8a16_direct(x, 4, 256, wq, s, 256, 64, None)
+    assert len(made) == 1 and not free
+    assert ops.linear_w8a16_direct(x, 4, 256, wq, s, 256, 64, None)[1] and len(made) == 2
+    torch.cuda.synchronize()   # (before the flags of this test go)
