@@ -34,11 +34,11 @@ template <> struct Kind<0> { typedef v4i Acc; };
 template <> struct Kind<1> { typedef v4f Acc; };
 template <> struct Kind<2> { typedef v4f Acc; };
 
-template <int NW, int TM, int TN, int NRG, int NCG, int RA, int BUDGET>
+template <int NW, int TM, int TN, int NRG, int NCG, int BUDGET>
 struct Cfg {
     static constexpr int KH = NW / (NRG * NCG);          // waves that split K
     static constexpr int BM = 16 * TM * NRG, BN = 16 * TN * NCG;
-    static constexpr int RBA = RA ? RA : BM / 8, RBW = BN / 8;   // 8-row blocks loaded per K block
+    static constexpr int RBA = BM / 8, RBW = BN / 8;         // 8-row blocks loaded per K block
     static constexpr int TOT = KH * (RBA + RBW);             // 1 KB wave loads per iteration
     static constexpr int LI = (TOT + NW - 1) / NW;   // per wave
     static constexpr int BLKB = (BM + BN) * BLK;             // LDS bytes of a K block
@@ -53,10 +53,10 @@ struct Cfg {
 };
 
 // Waves per SIMD that the registers allow: accumulators, one or two sets of fragments, addresses.
-constexpr int min_waves(int nw, int tm, int tn, bool pipe)
+constexpr int min_waves(int tm, int tn, bool pipe)
 {
     const int regs = 4 * tm * tn + (pipe ? 2 : 1) * 8 * (tm + tn) + 44;
-    return regs <= 128 ? 4 : regs <= 168 && nw == 4 ? 3 : regs <= 256 ? 2 : 1;
+    return regs <= 128 ? 4 : regs <= 256 ? 2 : 1;
 }
 
 template <int D, int LI>
@@ -72,12 +72,12 @@ __device__ __forceinline__ void wait_left(int left)   // at most `left` iteratio
     });
 }
 
-template <int KIND, int NW, int TM, int TN, int NRG, int NCG, int RA, int BUDGET, bool PIPE, bool GATE>
-__global__ void __launch_bounds__(64 * NW, min_waves(NW, TM, TN, PIPE))
+template <int KIND, int NW, int TM, int TN, int NRG, int NCG, int BUDGET, bool PIPE, bool GATE>
+__global__ void __launch_bounds__(64 * NW, min_waves(TM, TN, PIPE))
 q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__restrict__ W, int64_t ldw, int M, int N,
                 int K, Q8Epi ep, int out, int act)
 {
-    using C = Cfg<NW, TM, TN, NRG, NCG, RA, BUDGET>;
+    using C = Cfg<NW, TM, TN, NRG, NCG, BUDGET>;
     using Acc = typename Kind<KIND>::Acc;
     constexpr int KH = C::KH, LI = C::LI, D = C::D;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -135,7 +135,7 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
         const int e = 64 * c + lane;
         lds_ptr d = (lds_ptr)(ops + 64 * c);
         if (e < C::BM) {
-            if (ep.a_scale) __builtin_amdgcn_global_load_lds((glb_ptr)(ep.a_scale + min(m0 + e, M - 1)), d, 4, 0, 0);
+            __builtin_amdgcn_global_load_lds((glb_ptr)(ep.a_scale + min(m0 + e, M - 1)), d, 4, 0, 0);
         } else if (e < C::BM + 2 * C::BN) {
             const int wr = (e - C::BM) % C::BN;
             int n;
@@ -146,7 +146,7 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
                 n = min(n0 + wr, N - 1);
             }
             if (e < C::BM + C::BN) {
-                if (ep.w_scale) __builtin_amdgcn_global_load_lds((glb_ptr)(ep.w_scale + (ep.w_per_row ? n : 0)), d, 4, 0, 0);
+                __builtin_amdgcn_global_load_lds((glb_ptr)(ep.w_scale + (ep.w_per_row ? n : 0)), d, 4, 0, 0);
             } else if (ep.bias) {
                 if (ep.bias_dtype == PSQ_F32) __builtin_amdgcn_global_load_lds((glb_ptr)((const uint32_t *)ep.bias + n), d, 4, 0, 0);
                 else __builtin_amdgcn_global_load_lds((glb_ptr)((const uint16_t *)ep.bias + n), d, 2, 0, 0);
@@ -315,7 +315,7 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
                 const v4i wv = *(const v4i *)(ops + C::BM + wr), bv = *(const v4i *)(ops + C::BM + C::BN + wr);
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    ws[g][c] = ep.w_scale ? __int_as_float(wv[c]) : 1.0f;
+                    ws[g][c] = __int_as_float(wv[c]);
                     bs[g][c] = ep.bias ? bias_word((uint32_t)bv[c], ep.bias_dtype) : 0.0f;
                 }
             }
@@ -323,7 +323,7 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
             for (int i = 0; i < TM; i++) {
                 const int m = mb + 16 * i + fr;
                 if ((KH > 1 && i % KH != kh) || m >= M) continue;
-                const float as = ep.a_scale ? __uint_as_float(ops[rg * TM * 16 + 16 * i + fr]) : 1.0f;
+                const float as = __uint_as_float(ops[rg * TM * 16 + 16 * i + fr]);
                 float v[4];
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
@@ -372,11 +372,11 @@ q8_small_kernel(const uint8_t *__restrict__ A, int64_t lda, const uint8_t *__res
     }
 }
 
-template <int KIND, int NW, int TM, int TN, int NRG, int NCG, int RA, int BUDGET, bool PIPE, bool GATE>
+template <int KIND, int NW, int TM, int TN, int NRG, int NCG, int BUDGET, bool PIPE, bool GATE>
 int launch_cfg(int out, int act, const Q8Args &x)
 {
-    using C = Cfg<NW, TM, TN, NRG, NCG, RA, BUDGET>;
-    auto kern = q8_small_kernel<KIND, NW, TM, TN, NRG, NCG, RA, BUDGET, PIPE, GATE>;
+    using C = Cfg<NW, TM, TN, NRG, NCG, BUDGET>;
+    auto kern = q8_small_kernel<KIND, NW, TM, TN, NRG, NCG, BUDGET, PIPE, GATE>;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return set_error(PSQ_E_DEVICE, "%s: no device", x.name);
     static bool attr_set[64] = {};   // per device; the attribute is idempotent
@@ -418,7 +418,7 @@ int pick_shape(bool gate, int64_t M, int64_t N, int cus)
     const Shape *sh = gate ? kGateShapes : kShapes;
     auto tiles = [&](int i) { return ((M + sh[i].bm - 1) / sh[i].bm) * ((N + sh[i].bn - 1) / sh[i].bn); };
     if (M <= 16) return T16x32;
-    if (tiles(T16x32) <= cus * (sh[T16x32].wide ? 2 : 1)) return T16x32;
+    if (tiles(T16x32) <= 2 * cus) return T16x32;
     if (M <= 32 || tiles(T32x64) <= cus) return T32x64;
     if (tiles(T64x64) <= cus) return T64x64;
     if (sh[T80x64].bm && tiles(T80x64) <= cus) return T80x64;
@@ -436,25 +436,25 @@ int launch_shape(int shape, bool gate, int out, int act, const Q8Args &x)
     if (gate) {
         if constexpr (KIND != 2) {
             switch (shape) {
-            case T16x32: PSQ_GO(8, 1, 2, 1, 2, 0, 80 * KB, false, true);
-            case T32x64: PSQ_GO(8, 2, 2, 1, 4, 0, 156 * KB, false, true);
-            case T64x64: PSQ_GO(8, 4, 2, 1, 4, 0, 156 * KB, true, true);
-            case T96x128: PSQ_GO(8, 3, 2, 2, 4, 0, 156 * KB, true, true);
-            case T128x128: PSQ_GO(8, 4, 2, 2, 4, 0, 156 * KB, true, true);
-            default: PSQ_GO(8, 4, 4, 4, 2, 0, 156 * KB, true, true);
+            case T16x32: PSQ_GO(8, 1, 2, 1, 2, 80 * KB, false, true);
+            case T32x64: PSQ_GO(8, 2, 2, 1, 4, 156 * KB, false, true);
+            case T64x64: PSQ_GO(8, 4, 2, 1, 4, 156 * KB, true, true);
+            case T96x128: PSQ_GO(8, 3, 2, 2, 4, 156 * KB, true, true);
+            case T128x128: PSQ_GO(8, 4, 2, 2, 4, 156 * KB, true, true);
+            default: PSQ_GO(8, 4, 4, 4, 2, 156 * KB, true, true);
             }
         }
         return set_error(PSQ_E_ARG, "%s: no gate for these weights", x.name);
     }
     switch (shape) {
-    case T16x32: PSQ_GO(8, 1, 1, 1, 2, 0, 76 * KB, false, false);
-    case T32x64: PSQ_GO(8, 2, 1, 1, 4, 0, 76 * KB, false, false);
-    case T64x64: PSQ_GO(8, 4, 1, 1, 4, 0, 156 * KB, true, false);
-    case T80x64: PSQ_GO(8, 5, 1, 1, 4, 0, 156 * KB, true, false);
-    case T96x128: PSQ_GO(8, 3, 2, 2, 4, 0, 156 * KB, true, false);
-    case T128x128: PSQ_GO(8, 4, 2, 2, 4, 0, 156 * KB, true, false);
-    case T128x192: PSQ_GO(8, 4, 3, 2, 4, 0, 156 * KB, true, false);
-    default: PSQ_GO(8, 4, 4, 4, 2, 0, 156 * KB, true, false);
+    case T16x32: PSQ_GO(8, 1, 1, 1, 2, 76 * KB, false, false);
+    case T32x64: PSQ_GO(8, 2, 1, 1, 4, 76 * KB, false, false);
+    case T64x64: PSQ_GO(8, 4, 1, 1, 4, 156 * KB, true, false);
+    case T80x64: PSQ_GO(8, 5, 1, 1, 4, 156 * KB, true, false);
+    case T96x128: PSQ_GO(8, 3, 2, 2, 4, 156 * KB, true, false);
+    case T128x128: PSQ_GO(8, 4, 2, 2, 4, 156 * KB, true, false);
+    case T128x192: PSQ_GO(8, 4, 3, 2, 4, 156 * KB, true, false);
+    default: PSQ_GO(8, 4, 4, 4, 2, 156 * KB, true, false);
     }
 #undef PSQ_GO
 }
