@@ -39,14 +39,16 @@ struct WArgs {
     int sk = 0;
     float *part = nullptr;      // [2 sk][BM][256] fp32: the first and the last partial of each workgroup
     uint32_t *cnt = nullptr;    // [tiles] finished workgroups per tile: zero at launch, left zero
-    // int8: *flag = ticket when an output is NaN or +-Inf (null: not checked)
+    // int8, CHECK kernels: *flag = ticket when an output is NaN or +-Inf
     unsigned long long *flag = nullptr;
     unsigned long long ticket = 0;
 };
 
 // Collects whether any stored output is NaN or +-Inf: the exponent of every element, plus its lowest
 // bit, carries into bits 15 / 31 when it is all ones.  Three VALU ops per two 16-bit outputs beside the
-// store (of a checked call), where a pass over the finished output cost 5.8 us at 1024 x 5120 and a launch.
+// store, where a pass over the finished output cost 5.8 us at 1024 x 5120 and a launch.  Checked calls
+// have kernels of their own (CHECK): tests of the flag in one epilogue for both cost plain tiled calls
+// 0.6-0.7 us (the median of 68 sizes).
 struct Finite {
     uint32_t bad = 0;
     __device__ __forceinline__ void half2(uint32_t w, int dt)
@@ -69,7 +71,7 @@ struct Finite {
     __device__ __forceinline__ void report(const WArgs &wa) const
     {
         // a plain store (the flag may be host memory): the flag serves one call at a time, with growing tickets
-        if (wa.flag && (bad & 0x80008000u)) __hip_atomic_store(wa.flag, wa.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (bad & 0x80008000u) __hip_atomic_store(wa.flag, wa.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 };
 
@@ -153,7 +155,7 @@ __device__ __forceinline__ uint32_t i8pair_f16(uint32_t p, int hi)
     return __builtin_bit_cast(uint32_t, q);
 }
 
-template <int XDT, int WK, int MT>
+template <int XDT, int WK, int MT, bool CHECK>
 __global__ void __launch_bounds__(NTHREADS)
 gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int K, WArgs wa)
 {
@@ -274,10 +276,10 @@ gemm_wonly_skinny(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int
         const float cs = (WK == W_INT8) ? wa.scale32[nn] : 1.0f;
         const float bb = wa.bias ? load_elem(wa.bias, nn, wa.bias_dtype) : 0.0f;
         const float v = __builtin_fmaf(sum, cs, bb);
-        if (WK == W_INT8 && wa.flag) fin.store(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
+        if constexpr (CHECK) fin.store(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
         else store_elem(wa.y, (int64_t)m * wa.ldy + nn, wa.y_dtype, v);
     }
-    if constexpr (WK == W_INT8) fin.report(wa);
+    if constexpr (CHECK) fin.report(wa);
 }
 
 // ------------------------------------------------------------------ tiled kernel (M > 64)
@@ -348,7 +350,7 @@ __host__ __device__ inline int sk_slot(int l, int t, int64_t U, int G, int nk)
 }
 }  // namespace wt
 
-template <int XDT, int WK, int BM, bool SKM>
+template <int XDT, int WK, int BM, bool SKM, bool CHECK>
 __global__ void __launch_bounds__(wt::THREADS, 1)
 gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int K, WArgs wa)
 {
@@ -767,7 +769,7 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                         uint8_t *p = rowp[i] + (nc + 4 * h) * 2;
                         if (live[i]) {
                             *(v4i *)p = v4i{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
-                            if (WK == W_INT8 && wa.flag) {
+                            if constexpr (CHECK) {
 #pragma unroll
                                 for (int d = 0; d < 2; d++) {
                                     fin.half2(lo[d], wa.y_dtype);
@@ -791,7 +793,7 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                             constexpr int c = decltype(cc)::value;
                             const float v = value(i, j, 4 * g + c, cs[c], bs[c]);
                             if (live[i] && c < n_left0 - nc) {
-                                if (WK == W_INT8 && wa.flag) fin.store(rowp[i], nc + c, wa.y_dtype, v);
+                                if constexpr (CHECK) fin.store(rowp[i], nc + c, wa.y_dtype, v);
                                 else store_elem(rowp[i], nc + c, wa.y_dtype, v);
                             }
                         });
@@ -800,7 +802,7 @@ gemm_wonly_tiled(const uint16_t *__restrict__ x, int64_t ldx, int M, int N, int 
                 });
             });
         }
-        if constexpr (WK == W_INT8) fin.report(wa);
+        if constexpr (CHECK) fin.report(wa);
     }
 }
 
@@ -1808,24 +1810,24 @@ int launch_stream(const uint16_t *x, int64_t ldx, int64_t M, int64_t N, int64_t 
     return launch_stream_m<XDT, 4>(x, ldx, M, N, K, wa, st, name);
 }
 
-template <int XDT, int WK>
+template <int XDT, int WK, bool CHECK>
 void launch_skinny(const uint16_t *x, int64_t ldx, int64_t M, int64_t N, int64_t K, const WArgs &wa, hipStream_t st)
 {
     const dim3 grid((unsigned)((N + 15) / 16)), block(NTHREADS);
     const int mt = (int)((M + 15) / 16);
-    if (mt == 1) gemm_wonly_skinny<XDT, WK, 1><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
-    else if (mt == 2) gemm_wonly_skinny<XDT, WK, 2><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
-    else if (mt == 3) gemm_wonly_skinny<XDT, WK, 3><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
-    else gemm_wonly_skinny<XDT, WK, 4><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
+    if (mt == 1) gemm_wonly_skinny<XDT, WK, 1, CHECK><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
+    else if (mt == 2) gemm_wonly_skinny<XDT, WK, 2, CHECK><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
+    else if (mt == 3) gemm_wonly_skinny<XDT, WK, 3, CHECK><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
+    else gemm_wonly_skinny<XDT, WK, 4, CHECK><<<grid, block, 0, st>>>(x, ldx, (int)M, (int)N, (int)K, wa);
 }
 
 constexpr int64_t SKINNY_MAX_M = 64;   // largest M of the streaming and skinny kernels
 
-template <int XDT, int WK, int BM, bool SKM>
+template <int XDT, int WK, int BM, bool SKM, bool CHECK>
 int launch_tiled_bm(const uint16_t *x, int64_t ldx, int64_t M, int64_t N, int64_t K, const WArgs &wa, hipStream_t st,
                     const char *name)
 {
-    auto kern = gemm_wonly_tiled<XDT, WK, BM, SKM>;
+    auto kern = gemm_wonly_tiled<XDT, WK, BM, SKM, CHECK>;
     constexpr int lds = wt::lds_bytes<WK, BM>() + (SKM ? 16 : 0);   // + the word that broadcasts a stream-K count
     static_assert(lds <= 163840, "LDS of the tiled kernel");
     int dev = 0;
@@ -1887,6 +1889,13 @@ int launch(const void *x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_
            void *workspace, int64_t ws_bytes, hipStream_t st, const char *name)
 {
     const uint16_t *xp = (const uint16_t *)x;
+    // f(whether the outputs are checked)
+    auto checked = [&](auto f) {
+        if constexpr (WK == W_INT8) {
+            if (wa.flag) return f(std::true_type{});
+        }
+        return f(std::false_type{});
+    };
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return set_error(PSQ_E_DEVICE, "%s: no device", name);
     Path path = choose_path(WK, ldx, M, N, K, wa.gs, workspace != nullptr, cu_count(dev));
@@ -1904,8 +1913,12 @@ int launch(const void *x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_
         return x_dtype == PSQ_BF16 ? launch_stream<PSQ_BF16>(xp, ldx, M, N, K, wa, st, name)
                                    : launch_stream<PSQ_F16>(xp, ldx, M, N, K, wa, st, name);
     if (path == Path::Skinny) {
-        if (x_dtype == PSQ_BF16) launch_skinny<PSQ_BF16, WK>(xp, ldx, M, N, K, wa, st);
-        else launch_skinny<PSQ_F16, WK>(xp, ldx, M, N, K, wa, st);
+        checked([&](auto cc) {
+            constexpr bool CHECK = decltype(cc)::value;
+            if (x_dtype == PSQ_BF16) launch_skinny<PSQ_BF16, WK, CHECK>(xp, ldx, M, N, K, wa, st);
+            else launch_skinny<PSQ_F16, WK, CHECK>(xp, ldx, M, N, K, wa, st);
+            return PSQ_OK;
+        });
         return check_launch(name);
     }
     if (ldx > (1LL << 22)) return set_error(PSQ_E_SHAPE, "%s: ldx above 2^22", name);   // 32-bit row offsets
@@ -1923,14 +1936,17 @@ int launch(const void *x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_
     }
     auto go = [&](auto xc) {
         constexpr int XDT = decltype(xc)::value;
-        if (plan.sk) return launch_tiled_bm<XDT, WK, 128, true>(xp, ldx, M, N, K, wa, st, name);
-        switch (plan.bm) {
-        case 128: return launch_tiled_bm<XDT, WK, 128, false>(xp, ldx, M, N, K, wa, st, name);
-        case 160: return launch_tiled_bm<XDT, WK, 160, false>(xp, ldx, M, N, K, wa, st, name);
-        case 192: return launch_tiled_bm<XDT, WK, 192, false>(xp, ldx, M, N, K, wa, st, name);
-        case 224: return launch_tiled_bm<XDT, WK, 224, false>(xp, ldx, M, N, K, wa, st, name);
-        default: return launch_tiled_bm<XDT, WK, 256, false>(xp, ldx, M, N, K, wa, st, name);
-        }
+        return checked([&](auto cc) {
+            constexpr bool CHECK = decltype(cc)::value;
+            if (plan.sk) return launch_tiled_bm<XDT, WK, 128, true, CHECK>(xp, ldx, M, N, K, wa, st, name);
+            switch (plan.bm) {
+            case 128: return launch_tiled_bm<XDT, WK, 128, false, CHECK>(xp, ldx, M, N, K, wa, st, name);
+            case 160: return launch_tiled_bm<XDT, WK, 160, false, CHECK>(xp, ldx, M, N, K, wa, st, name);
+            case 192: return launch_tiled_bm<XDT, WK, 192, false, CHECK>(xp, ldx, M, N, K, wa, st, name);
+            case 224: return launch_tiled_bm<XDT, WK, 224, false, CHECK>(xp, ldx, M, N, K, wa, st, name);
+            default: return launch_tiled_bm<XDT, WK, 256, false, CHECK>(xp, ldx, M, N, K, wa, st, name);
+            }
+        });
     };
     return x_dtype == PSQ_BF16 ? go(std::integral_constant<int, PSQ_BF16>{}) : go(std::integral_constant<int, PSQ_F16>{});
 }
