@@ -323,16 +323,16 @@ def quantized_in_gemm(M, K, act):
 
 
 def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, act, into=None):
-    """x [..., K] contiguous bf16/f16; w, w_scale: device addresses.  [..., N] (gate: N / 2) of x's
-    dtype; into: [M, N] rows of x's dtype or fp32 (the same values) that take the result."""
+    """x [..., K] contiguous bf16/f16; w, w_scale, bias (of x's dtype, or None): device addresses.
+    [..., N] (gate: N / 2) of x's dtype; into: [M, N] rows of x's dtype or fp32 (the same values) that
+    take the result."""
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
     y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device) if into is None else into
-    scratch = None if quantized_in_gemm(M, K, act) else \
+    scratch = None if M <= 2 and quantized_in_gemm(M, K, act) else \
         torch.empty(((M * K + 15) & -16) + 4 * M, dtype=torch.uint8, device=x.device)
     status = lib.psq_linear_q8(weights, x.data_ptr(), dt, K, rot_group, w, K, w_scale, per_row,
-                               None if bias is None else bias.data_ptr(), dt, act, y.data_ptr(),
-                               int(y.dtype is torch.float32), cols, M, N, K,
+                               bias, dt, act, y.data_ptr(), int(y.dtype is torch.float32), cols, M, N, K,
                                None if scratch is None else scratch.data_ptr(),
                                _raw_stream(x.device.index))
     return None if status else y
@@ -353,25 +353,24 @@ def linear_codes_direct(x, q, scale, M, K, weights, w, w_scale, per_row, N, bias
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
     y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device)
-    b = None if bias is None else bias.data_ptr()
     out = (y.data_ptr(), dt, cols, M, N, K, _raw_stream(x.device.index))
     if weights == _native.Q8_I8:
-        status = lib.psq_gemm_i8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, b, dt, act, *out)
+        status = lib.psq_gemm_i8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, bias, dt, act, *out)
     elif weights == _native.Q8_E4M3:
-        status = lib.psq_gemm_fp8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, b, dt, act, *out)
+        status = lib.psq_gemm_fp8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, bias, dt, act, *out)
     else:
-        status = lib.psq_gemm_fp8_e5m2w(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, b, dt, *out)
+        status = lib.psq_gemm_fp8_e5m2w(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, bias, dt, *out)
     return None if status else y
 
 
 def linear_w4a16_direct(x, M, K, wq, w_scale, w_zero, group_size, N, bias, into=None):
-    """x [..., K] contiguous bf16/f16; wq, w_scale, w_zero: device addresses.  [..., N]; into: [M, N]
-    rows of x's dtype that take the result."""
+    """x [..., K] contiguous bf16/f16; wq, w_scale, w_zero, bias (of x's dtype, or None): device
+    addresses.  [..., N]; into: [M, N] rows of x's dtype that take the result."""
     lib, dt, stream = _native.lib(), _DT[x.dtype], _raw_stream(x.device.index)
     ws, nb = _workspace(x.device, stream or None, lib.psq_gemm_wonly_workspace_bytes(_native.W_UINT4, K, M, N, K, group_size))
     y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device) if into is None else into
     status = lib.psq_gemm_w4a16_ws(x.data_ptr(), dt, K, wq, w_scale, w_zero, group_size,
-                                   None if bias is None else bias.data_ptr(), dt, y.data_ptr(), dt, N, M, N, K,
+                                   bias, dt, y.data_ptr(), dt, N, M, N, K,
                                    None if ws is None else ws.data_ptr(), nb, stream)
     return None if status else y
 
@@ -389,21 +388,18 @@ _flags_lock = threading.Lock()
 
 
 def _take_flag(index):
+    """[flag tensor, last ticket, flag word, the list it goes back to]"""
+    try:
+        return _host_flags[index][1].pop()   # (pop and append are one step each: no lock)
+    except (KeyError, IndexError):
+        pass
     with _flags_lock:
         made, free = _host_flags.setdefault(index, ([], []))
-        if free:
-            return free.pop()
         if len(made) >= _MAX_FLAGS:
             return None
         flag = torch.zeros(1, dtype=torch.int64, pin_memory=True)
-        made.append([flag, 0, ctypes.c_uint64.from_address(flag.data_ptr())])
+        made.append([flag, 0, ctypes.c_uint64.from_address(flag.data_ptr()), free])
         return made[-1]
-
-
-def _give_flag(index, entry):
-    with _flags_lock:
-        if index in _host_flags:
-            _host_flags[index][1].append(entry)
 
 
 def linear_w8a16_launch(x, M, K, wq, w_scale, rot_group, N, bias):
@@ -424,7 +420,7 @@ def linear_w8a16_launch(x, M, K, wq, w_scale, rot_group, N, bias):
             y.data_ptr(), N, M, N, K, None if rotated is None else rotated.data_ptr(),
             None if ws is None else ws.data_ptr(), nb, entry[0].data_ptr(), ticket, stream), "linear_w8a16")
     except Exception:   # refused: the GEMM was not launched
-        _give_flag(device.index, entry)
+        entry[3].append(entry)
         raise
     return y, (device, entry, ticket)
 
@@ -435,7 +431,7 @@ def linear_w8a16_finite(check):
     device, entry, ticket = check
     torch.cuda.current_stream(device).synchronize()
     finite = entry[2].value < ticket
-    _give_flag(device.index, entry)
+    entry[3].append(entry)
     return finite
 
 
