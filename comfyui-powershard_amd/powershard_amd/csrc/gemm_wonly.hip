@@ -8,8 +8,9 @@
 // W8A16: int8 values are exact in bf16, the per-row scale is applied in the epilogue,
 // y = round_out(fmaf(acc, s[n], bias[n])) (Int8Linear storage, powershard/operations.py:96-132).
 //
-// Two kernels: a weight-streaming one for M <= 64 (decode / short prompts: HBM-bound) and a
-// 256 x 256-tile one for larger M (MFMA-bound), both described where they are defined.
+// Kernels, each described where it is defined: uint4 decode (M <= 8) and weight streaming (M <= 64),
+// bound by the weight stream and the dequantization; the skinny one for M <= 64 otherwise; and the tiled
+// one, row tiles of 128 to 256 by 256 columns, for larger M.
 #include "psq_common.hpp"
 #include "wonly_plan.hpp"
 
