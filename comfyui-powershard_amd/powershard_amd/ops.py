@@ -323,16 +323,16 @@ def quantized_in_gemm(M, K, act):
 
 
 def linear_q8_direct(x, M, K, weights, w, w_scale, per_row, rot_group, N, bias, act, into=None):
-    """x [..., K] contiguous bf16/f16; w, w_scale, bias (of x's dtype, or None): device addresses.
-    [..., N] (gate: N / 2) of x's dtype; into: [M, N] rows of x's dtype or fp32 (the same values) that
-    take the result."""
+    """x [..., K] contiguous bf16/f16; w, w_scale: device addresses.  [..., N] (gate: N / 2) of x's
+    dtype; into: [M, N] rows of x's dtype or fp32 (the same values) that take the result."""
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
     y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device) if into is None else into
     scratch = None if M <= 2 and quantized_in_gemm(M, K, act) else \
         torch.empty(((M * K + 15) & -16) + 4 * M, dtype=torch.uint8, device=x.device)
     status = lib.psq_linear_q8(weights, x.data_ptr(), dt, K, rot_group, w, K, w_scale, per_row,
-                               bias, dt, act, y.data_ptr(), int(y.dtype is torch.float32), cols, M, N, K,
+                               None if bias is None else bias.data_ptr(), dt, act, y.data_ptr(),
+                               int(y.dtype is torch.float32), cols, M, N, K,
                                None if scratch is None else scratch.data_ptr(),
                                _raw_stream(x.device.index))
     return None if status else y
@@ -353,24 +353,25 @@ def linear_codes_direct(x, q, scale, M, K, weights, w, w_scale, per_row, N, bias
     lib, dt = _native.lib(), _DT[x.dtype]
     cols = _out_cols(N, act, "linear_q8")
     y = torch.empty(x.shape[:-1] + (cols,), dtype=x.dtype, device=x.device)
+    b = None if bias is None else bias.data_ptr()
     out = (y.data_ptr(), dt, cols, M, N, K, _raw_stream(x.device.index))
     if weights == _native.Q8_I8:
-        status = lib.psq_gemm_i8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, bias, dt, act, *out)
+        status = lib.psq_gemm_i8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, b, dt, act, *out)
     elif weights == _native.Q8_E4M3:
-        status = lib.psq_gemm_fp8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, bias, dt, act, *out)
+        status = lib.psq_gemm_fp8_act(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, b, dt, act, *out)
     else:
-        status = lib.psq_gemm_fp8_e5m2w(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, bias, dt, *out)
+        status = lib.psq_gemm_fp8_e5m2w(q.data_ptr(), K, scale.data_ptr(), w, K, w_scale, per_row, b, dt, *out)
     return None if status else y
 
 
 def linear_w4a16_direct(x, M, K, wq, w_scale, w_zero, group_size, N, bias, into=None):
-    """x [..., K] contiguous bf16/f16; wq, w_scale, w_zero, bias (of x's dtype, or None): device
-    addresses.  [..., N]; into: [M, N] rows of x's dtype that take the result."""
+    """x [..., K] contiguous bf16/f16; wq, w_scale, w_zero: device addresses.  [..., N]; into: [M, N]
+    rows of x's dtype that take the result."""
     lib, dt, stream = _native.lib(), _DT[x.dtype], _raw_stream(x.device.index)
     ws, nb = _workspace(x.device, stream or None, lib.psq_gemm_wonly_workspace_bytes(_native.W_UINT4, K, M, N, K, group_size))
     y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device) if into is None else into
     status = lib.psq_gemm_w4a16_ws(x.data_ptr(), dt, K, wq, w_scale, w_zero, group_size,
-                                   bias, dt, y.data_ptr(), dt, N, M, N, K,
+                                   None if bias is None else bias.data_ptr(), dt, y.data_ptr(), dt, N, M, N, K,
                                    None if ws is None else ws.data_ptr(), nb, stream)
     return None if status else y
 

@@ -361,7 +361,9 @@ class QuantLinear(nn.Module):
                 or not store.is_contiguous() or not ops.direct_available()):
             return None
         try:
-            base, start, bias_at = store.data_ptr(), x.data_ptr(), None if bias is None else bias.data_ptr()
+            base, start = store.data_ptr(), x.data_ptr()
+            if bias is not None:
+                bias.data_ptr()
         except RuntimeError:   # no memory of its own (vmap)
             return None
         M = numel // K
@@ -376,7 +378,7 @@ class QuantLinear(nn.Module):
                 return None
             if into is not None and (into.dtype is not dtype or not _takes(into, device, M, N)):
                 into = None
-            return ops.linear_w4a16_direct(x, M, K, base + q_at, base + s_at, base + z_at, group, N, bias_at, into)
+            return ops.linear_w4a16_direct(x, M, K, base + q_at, base + s_at, base + z_at, group, N, bias, into)
         weights, count, rot = _Q8_WEIGHTS.get(code), s_bytes // 4, 0
         if (weights is None or sdtype is not torch.float32 or (activation is not None and weights == 2)
                 or (activation == "silu_gate" and N % 128)):
@@ -397,8 +399,8 @@ class QuantLinear(nn.Module):
         if cache is not None and into is None and not ops.quantized_in_gemm(M, K, act):
             codes = _shared_codes(cache, x, M, K, weights != 0, rot)
             return None if codes is None else ops.linear_codes_direct(
-                x, *codes, M, K, weights, base + q_at, base + s_at, int(count > 1), N, bias_at, act)
-        return ops.linear_q8_direct(x, M, K, weights, base + q_at, base + s_at, int(count > 1), rot, N, bias_at, act, into)
+                x, *codes, M, K, weights, base + q_at, base + s_at, int(count > 1), N, bias, act)
+        return ops.linear_q8_direct(x, M, K, weights, base + q_at, base + s_at, int(count > 1), rot, N, bias, act, into)
 
     def _forward(self, x, activation, into=None):
         if self._ps_native:
